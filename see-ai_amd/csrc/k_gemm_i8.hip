@@ -14,22 +14,17 @@
 // QWt [N, K] (K contiguous: both MFMA operands then read 16 contiguous
 // bytes per lane).
 //
-// Large M (M, N >= the tile policy's w8a8_large_min, 4096 by default; K a
-// multiple of 64): GemmI8DmaKernel, a 256 x 256
-// tile per workgroup of eight waves (two per SIMD, blocks of 128 x 64 on
-// v_mfma_i32_32x32x32_i8), K staged 64 bytes at a time through four LDS
-// buffers filled by direct-to-LDS buffer loads, three stages in flight;
-// workgroups are ordered so each XCD's L2 serves a compact block of tiles.
-// Other large shapes: GemmI8TileKernel (sixteen waves of 64 x 64, loads
-// staged through registers into two padded LDS buffers).
-// Small M (decode-like, M <= 64): one 16-column slice of C per workgroup,
-// its four waves each reducing a quarter of K on v_mfma_i32_16x16x64_i8
-// straight from global memory (each weight byte is read once), then summed
-// through LDS -- the weight stream is the whole cost, spread over N/16
-// workgroups.
+// K a multiple of 16 (and the operands 16-byte aligned): GemmI8DmaKernel, K
+// staged 64 bytes at a time through LDS buffers filled by direct-to-LDS buffer
+// loads, several stages in flight, on v_mfma_i32_32x32x32_i8.  Its tile goes
+// from 256 x 256 (eight waves, a prefill batch) down to 32 x 32 with K split
+// over four wave groups of the workgroup (decode, M <= 64): PickTile has the
+// rule.  Other K or alignments: GemmI8TileKernel with unaligned loads, staged
+// through registers into two padded LDS buffers.
 #include <algorithm>
 #include <atomic>
 #include <cfloat>
+#include <cmath>
 #include <cstdlib>
 
 #include "common.h"
@@ -303,16 +298,40 @@ __device__ __forceinline__ void TileOf(int b, int tiles_m, int tiles_n, int& tm,
   tn = off / rows;
 }
 
+// 16 bytes of a row: rows of 16-byte multiples are read aligned (kAl), others
+// with loads marked unaligned.
+template <bool kAl>
+__device__ __forceinline__ v4i LoadChunk(const int8_t* p) {
+  if constexpr (kAl) {
+    return *reinterpret_cast<const v4i*>(p);
+  } else {
+    typedef int v4iu __attribute__((ext_vector_type(4), aligned(1)));
+    return *reinterpret_cast<const v4iu*>(p);
+  }
+}
+
+// 16 bytes of a row from its byte k, bytes at K and past it zero.
+__device__ __forceinline__ v4i LoadTail(const int8_t* row, int64_t k, int64_t K) {
+  if (k + 16 <= K) return LoadChunk<false>(row + k);
+  v4i v = {0, 0, 0, 0};
+  for (int e = 0; e < 16 && k + e < K; ++e)
+    v[e / 4] |= static_cast<int>(static_cast<uint32_t>(static_cast<uint8_t>(row[k + e])) << (8 * (e % 4)));
+  return v;
+}
+
 // BM x BN tile per workgroup of WGM x WGN waves, each wave a (BM/WGM) x
 // (BN/WGN) block of 32 x 32 x 32 int8 MFMAs.  K advances BK bytes per step
 // through two LDS buffers (rows padded by 16 bytes): the next step's global
 // loads are issued before the current step's MFMAs and land in the other
-// buffer after them, so one barrier per step orders both hazards.
-template <int BM, int BN, int BK, int WGM, int WGN>
+// buffer after them, so one barrier per step orders both hazards.  Without
+// kAl, rows of any length and alignment: unaligned loads, the last step's
+// bytes past K masked to zero.
+template <int BM, int BN, int BK, int WGM, int WGN, bool kAl>
 __global__ void __launch_bounds__(WGM * WGN * kWave)
 GemmI8TileKernel(const int8_t* __restrict__ QA, const float* __restrict__ sa,
                  const int8_t* __restrict__ QW, const float* __restrict__ sw,
-                 float* __restrict__ C, int32_t* __restrict__ acc_out, int M, int N, int K) {
+                 float* __restrict__ C, int32_t* __restrict__ acc_out, int M, int N, int64_t K,
+                 size_t ldc) {
   constexpr int kT = WGM * WGN * kWave;        // lanes per workgroup
   constexpr int LDK = BK + 16;                 // padded LDS row stride (bytes)
   constexpr int WM = BM / WGM, WN = BN / WGN;  // per-wave block
@@ -343,22 +362,27 @@ GemmI8TileKernel(const int8_t* __restrict__ QA, const float* __restrict__ sa,
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
 
   v4i ra[NA], rb[NB];
-  auto load = [&](int k0) {
+  auto load = [&](int64_t k0) {
+    const bool whole = k0 + BK <= K;  // wave-uniform
 #pragma unroll
     for (int e = 0; e < NA; ++e) {
       const int c = tid + e * kT;
-      const int row = c / kChunksRow, kc = c % kChunksRow;
-      const int m = m0 + row, k = k0 + kc * 16;
-      ra[e] = (m < M && k < K) ? *reinterpret_cast<const v4i*>(QA + static_cast<size_t>(m) * K + k)
-                               : v4i{0, 0, 0, 0};
+      const int m = m0 + c / kChunksRow;
+      const int64_t k = k0 + c % kChunksRow * 16;
+      const int8_t* row = QA + static_cast<size_t>(m) * K;
+      ra[e] = !(m < M) || k >= K ? v4i{0, 0, 0, 0}
+              : kAl || whole      ? LoadChunk<kAl>(row + k)
+                                  : LoadTail(row, k, K);
     }
 #pragma unroll
     for (int e = 0; e < NB; ++e) {
       const int c = tid + e * kT;
-      const int row = c / kChunksRow, kc = c % kChunksRow;
-      const int n = n0 + row, k = k0 + kc * 16;
-      rb[e] = (n < N && k < K) ? *reinterpret_cast<const v4i*>(QW + static_cast<size_t>(n) * K + k)
-                               : v4i{0, 0, 0, 0};
+      const int n = n0 + c / kChunksRow;
+      const int64_t k = k0 + c % kChunksRow * 16;
+      const int8_t* row = QW + static_cast<size_t>(n) * K;
+      rb[e] = !(n < N) || k >= K ? v4i{0, 0, 0, 0}
+              : kAl || whole      ? LoadChunk<kAl>(row + k)
+                                  : LoadTail(row, k, K);
     }
   };
   auto store = [&](int buf) {
@@ -374,7 +398,7 @@ GemmI8TileKernel(const int8_t* __restrict__ QA, const float* __restrict__ sa,
     }
   };
 
-  const int nsteps = (K + BK - 1) / BK;
+  const int nsteps = static_cast<int>((K + BK - 1) / BK);
   constexpr int KS = BK / 32;  // 32-byte k-steps per LDS buffer
   v4i af[2][TM], bf[2][TN];
   auto read_frags = [&](int buf, int ks, int slot) {
@@ -391,7 +415,7 @@ GemmI8TileKernel(const int8_t* __restrict__ QA, const float* __restrict__ sa,
   __syncthreads();
   for (int it = 0; it < nsteps; ++it) {
     const int buf = it & 1;
-    if (it + 1 < nsteps) load((it + 1) * BK);
+    if (it + 1 < nsteps) load(static_cast<int64_t>(it + 1) * BK);
     // Fragments double-buffered in registers: the next k-step's LDS reads
     // are in flight while the current k-step's MFMAs issue.
     read_frags(buf, 0, 0);
@@ -423,13 +447,13 @@ GemmI8TileKernel(const int8_t* __restrict__ QA, const float* __restrict__ sa,
         for (int r = 0; r < 16; ++r) {
           const int m = m0 + wm + i * 32 + 8 * (r / 4) + 4 * (lane / 32) + (r % 4);
           const int n = n0 + wn + j * 32 + lane % 32;
-          if (m < M && n < N) acc_out[static_cast<size_t>(m) * N + n] = acc[i][j][r];
+          if (m < M && n < N) acc_out[static_cast<size_t>(m) * ldc + n] = acc[i][j][r];
         }
   }
   constexpr int SLD = WN + 4;  // staging row stride (floats)
   static_assert(WGM * WGN * 32 * SLD * 4 <= 2 * (BM + BN) * LDK, "staging fits in LDS");
   float* stage = reinterpret_cast<float*>(smem) + wave * 32 * SLD;
-  const bool vec_out = (N % 4) == 0;
+  const bool vec_out = ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
   float swv[TN];
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
@@ -443,7 +467,7 @@ GemmI8TileKernel(const int8_t* __restrict__ QA, const float* __restrict__ sa,
     for (int q = 0; q < 4; ++q) {
       const int m4 = mb + 8 * q + 4 * (lane / 32);
       float sav[4];
-      if (m4 + 3 < M && (M % 4) == 0) {
+      if (kAl && m4 + 3 < M && (M % 4) == 0) {
         const float4 v = *reinterpret_cast<const float4*>(sa + m4);
         sav[0] = v.x, sav[1] = v.y, sav[2] = v.z, sav[3] = v.w;
       } else {
@@ -468,7 +492,7 @@ GemmI8TileKernel(const int8_t* __restrict__ QA, const float* __restrict__ sa,
       const int m = mb + row, n = n0 + wn + c4 * 4;
       const float4 v = *reinterpret_cast<const float4*>(stage + row * SLD + c4 * 4);
       if (m >= M) continue;
-      float* dst = C + static_cast<size_t>(m) * N + n;
+      float* dst = C + static_cast<size_t>(m) * ldc + n;
       if (vec_out && n + 3 < N) {
         *reinterpret_cast<float4*>(dst) = v;
       } else {
@@ -482,28 +506,37 @@ GemmI8TileKernel(const int8_t* __restrict__ QA, const float* __restrict__ sa,
   }
 }
 
-// --- the large-M GEMM, staged by direct-to-LDS loads -----------------------------
+// --- the GEMM staged by direct-to-LDS loads ---------------------------------------
 //
-// 256 x 256 tile per workgroup of WGM x WGN waves, each a (256/WGM) x
-// (256/WGN) block of v_mfma_i32_32x32x32_i8 accumulators.  The launcher runs
-// eight waves (two per SIMD, 2 x 4, blocks of 128 x 64: 128 int32
-// accumulators per lane), measured 6-7 % faster than four waves of 128 x 128
-// (one per SIMD, 256 accumulators) at 4096^3 and 8192^3: the second wave on
-// each SIMD issues MFMAs while the first waits on LDS or the barrier.  K moves 64 bytes per stage through kStages LDS buffers (32 KiB
-// each: 256 A rows + 256 W rows of 64 bytes) filled by buffer_load ... lds,
+// BM x BN tile per workgroup of KG k-groups of WGM x WGN waves, each wave a
+// (BM/WGM) x (BN/WGN) block of v_mfma_i32_32x32x32_i8 accumulators over its
+// group's K / KG.  K moves 64 bytes per stage through each group's kStages LDS
+// buffers (BM A rows + BN W rows of 64 bytes) filled by buffer_load ... lds,
 // which writes a wave's 64 x 16 bytes to consecutive LDS addresses from M0
 // without passing through registers; kStages - 1 stages are in flight while
 // one is multiplied.  One barrier per stage: every wave's loads of the
 // stage it is about to read have landed (vmcnt), and every wave has
 // finished reading the buffer the next load overwrites.
 //
+// The 256 x 256 tile runs eight waves (two per SIMD, 2 x 4, blocks of 128 x
+// 64: 128 int32 accumulators per lane), measured 6-7 % faster than four waves
+// of 128 x 128 (one per SIMD, 256 accumulators) at 4096^3 and 8192^3: the
+// second wave on each SIMD issues MFMAs while the first waits on LDS or the
+// barrier.  Small tiles are bound by the latency of their stages' loads, which
+// is why K splits over groups there: four groups walk a quarter of the stages
+// each with four times the loads in flight, and their int32 partials add
+// through LDS (exact in any order).  32 x 4096 x 4096: 9.2 us on fragments
+// straight from global memory (16 rows of 64 bytes an instruction), 7.0 us
+// here; 256 x 4096 x 4096: 31.5 us on register-staged 128 x 128 tiles, 13.2
+// us on 64 x 64 with two groups.
+//
 // LDS rows are 64 bytes, four 16-byte chunks; chunk c of row r sits at
 // physical chunk (c + r/4) mod 4.  The fragment reads (lane l: row l % 32,
 // chunk 2ks + l / 32) are then free of bank conflicts -- measured with
 // SQ_LDS_BANK_CONFLICT on gfx950 for ds_read_b128, which also counts
 // conflicts for rotations that bring in r/8 or r/16.  Loads pick the global
-// chunk that belongs at each physical slot.  Rows past M (or N) read as zeros (buffer
-// range check); K must be a multiple of 64.
+// chunk that belongs at each physical slot.  Rows past M (or N) and chunks
+// past K read as zeros (buffer range check); K must be a multiple of 16.
 constexpr int kDmaBK = 64;
 constexpr int kDmaChunks = kDmaBK / 16;
 
@@ -519,31 +552,35 @@ __device__ __forceinline__ void WaitVm() {
   __builtin_amdgcn_s_waitcnt((n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14));
 }
 
-template <int kStages, int WGM, int WGN>
-__global__ void __launch_bounds__(WGM * WGN * kWave)
+template <int BM, int BN, int kStages, int WGM, int WGN, int KG, bool kTail = true>
+__global__ void __launch_bounds__(KG * WGM * WGN * kWave)
 GemmI8DmaKernel(const int8_t* __restrict__ QA, const float* __restrict__ sa,
                 const int8_t* __restrict__ QW, const float* __restrict__ sw,
                 float* __restrict__ C, int32_t* __restrict__ acc_out, int M, int N, int K) {
-  constexpr int BM = 256, BN = 256;
-  constexpr int kWaves = WGM * WGN;
+  constexpr int kWaves = WGM * WGN;                 // waves of one k-group
   constexpr int WM = BM / WGM, WN = BN / WGN;       // per-wave block
   constexpr int TM = WM / 32, TN = WN / 32;         // 32 x 32 accumulators per wave
   constexpr int kRowsPerLoad = kWave / kDmaChunks;  // rows one wave-load fills (16)
-  constexpr int kLoads = BM / kRowsPerLoad / kWaves;  // wave-loads per operand, stage, wave
-  static_assert(kLoads * kRowsPerLoad * kWaves == BM, "loads cover the tile");
+  constexpr int kLoadsA = BM / kRowsPerLoad / kWaves;  // wave-loads per stage and wave
+  constexpr int kLoadsB = BN / kRowsPerLoad / kWaves;
+  static_assert(kTail || KG == 1, "one group");
+  static_assert(kLoadsA * kRowsPerLoad * kWaves == BM && kLoadsB * kRowsPerLoad * kWaves == BN,
+                "loads cover the tile");
   constexpr int kStageA = BM * kDmaBK;               // bytes
   constexpr int kStage = (BM + BN) * kDmaBK;
-  constexpr int kPerStage = 2 * kLoads;              // vmcnt units per stage
-  __shared__ __attribute__((aligned(1024))) int8_t smem[kStages * kStage];
+  constexpr int kPerStage = kLoadsA + kLoadsB;       // vmcnt units per stage
+  __shared__ __attribute__((aligned(1024))) int8_t smem_all[KG * kStages * kStage];
 
   const int tid = threadIdx.x;
-  const int wave = tid / kWave, lane = tid % kWave;
+  const int wave_wg = tid / kWave, lane = tid % kWave;
+  const int wave = wave_wg % kWaves, kg = KG > 1 ? Uniform(wave_wg / kWaves) : 0;
+  int8_t* const smem = smem_all + kg * (kStages * kStage);
   int tm, tn;
   TileOf(blockIdx.x, (M + BM - 1) / BM, (N + BN - 1) / BN, tm, tn);
   const int m0 = tm * BM, n0 = tn * BN;
 
   // Operand ranges start at this tile's first row: offsets stay below
-  // 256 * K, and rows past the operand's end fall outside num_records.
+  // BM * K, and rows past the operand's end fall outside num_records.
   const __amdgpu_buffer_rsrc_t rs_a = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<int8_t*>(QA) + static_cast<size_t>(m0) * K, 0,
       Uniform((M - m0) * K), 0x00020000);
@@ -551,28 +588,40 @@ GemmI8DmaKernel(const int8_t* __restrict__ QA, const float* __restrict__ sa,
       const_cast<int8_t*>(QW) + static_cast<size_t>(n0) * K, 0,
       Uniform((N - n0) * K), 0x00020000);
   // This lane's slot in each wave-load: row rbase + lane / 4, physical chunk
-  // lane % 4, which holds logical chunk (p - r/4) mod 4.
+  // lane % 4, which holds logical chunk (p - r/4) mod 4 (the same for all of
+  // its rows: they differ by multiples of 16).
   // (Fixed capacity: an array sized by a template-dependent constant and
   // captured by the lambdas below loses the kernel's host-side stub.)
-  static_assert(kLoads <= 4, "voff capacity");
+  static_assert(kLoadsA <= 4 && kLoadsB <= 4, "voff capacity");
+  constexpr int kLoads = kLoadsA > kLoadsB ? kLoadsA : kLoadsB;
   int voff[4];
+  const int chunk = ((lane % kDmaChunks - (lane / kDmaChunks) / 4) & 3) * 16;
 #pragma unroll
-  for (int j = 0; j < kLoads; ++j) {
-    const int row = (j * kWaves + wave) * kRowsPerLoad + lane / kDmaChunks;
-    const int c = (lane % kDmaChunks - row / 4) & 3;
-    voff[j] = row * K + c * 16;
-  }
+  for (int j = 0; j < kLoads; ++j)
+    voff[j] = ((j * kWaves + wave) * kRowsPerLoad + lane / kDmaChunks) * K + chunk;
+  // This k-group's stages: [kg T, kg T + T) of the K / 64 (rounded up); a
+  // chunk at K or past it is read from outside the operand's range, which
+  // leaves zeros in LDS.  Without kTail (K % 64 == 0, one group) every stage
+  // is whole and its offset stays scalar: the per-lane select costs the 256 x
+  // 256 tile 0.7 % at 4096^3.
+  const int nsteps_all = (K + kDmaBK - 1) / kDmaBK;
+  const int nsteps = (nsteps_all + KG - 1) / KG;
+  const int kbase = kg * nsteps * kDmaBK;
   auto issue = [&](int st, int buf) {
     int8_t* sA = smem + buf * kStage;
     int8_t* sB = sA + kStageA;
-    const int k0 = st * kDmaBK;
+    const int k0 = kbase + st * kDmaBK;
+    const int kadd = !kTail ? 0 : k0 + chunk < K ? k0 : INT32_MIN;
+    const int soff = kTail ? 0 : k0;
 #pragma unroll
     for (int j = 0; j < kLoads; ++j) {
       const int rbase = Uniform((j * kWaves + wave) * kRowsPerLoad);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_a, (LdsPtr)(sA + rbase * kDmaBK), 16, voff[j],
-                                               k0, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_b, (LdsPtr)(sB + rbase * kDmaBK), 16, voff[j],
-                                               k0, 0, 0);
+      if (j < kLoadsA)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_a, (LdsPtr)(sA + rbase * kDmaBK), 16,
+                                                 voff[j] + kadd, soff, 0, 0);
+      if (j < kLoadsB)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs_b, (LdsPtr)(sB + rbase * kDmaBK), 16,
+                                                 voff[j] + kadd, soff, 0, 0);
     }
   };
 
@@ -594,12 +643,10 @@ GemmI8DmaKernel(const int8_t* __restrict__ QA, const float* __restrict__ sa,
 
   // Software pipeline, one k-step (32 bytes of K) ahead in registers: while
   // the MFMAs of one k-step issue, the fragments of the next are read from
-  // LDS (interleaved two MFMAs per read).  The barrier sits between a
-  // stage's two k-steps: after it, stage it + 1 has landed, and every wave
-  // has consumed its reads of stage it - 1 (their MFMAs were issued before
-  // the barrier), whose buffer then takes the loads of stage
-  // it + kStages - 1.
-  const int nsteps = K / kDmaBK;
+  // LDS (spread over the MFMAs).  The barrier sits between a stage's two
+  // k-steps: after it, stage it + 1 has landed, and every wave has consumed
+  // its reads of stage it - 1 (their MFMAs were issued before the barrier),
+  // whose buffer then takes the loads of stage it + kStages - 1.
   v4i fa[2][TM], fb[2][TN];
   auto read = [&](int buf, int fo, int slot) {
     const int8_t* sA = smem + buf * kStage;
@@ -619,27 +666,20 @@ GemmI8DmaKernel(const int8_t* __restrict__ QA, const float* __restrict__ sa,
         acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[slot][j], fa[slot][i], acc[i][j],
                                                           0, 0, 0);
   };
-  // The next k-step's TM + TN LDS reads spread one per MFMA from the start
-  // of a k-step's TM x TN MFMAs; after the barrier, the stage's loads take
-  // the following MFMA slots.
-  auto interleave = [&]() {
+  // The next k-step's TM + TN LDS reads spread over a k-step's TM x TN MFMAs
+  // from its start; after the barrier, the stage's loads take the last MFMA
+  // slots.
+  constexpr int kMfmas = TM * TN, kReads = TM + TN;
+  constexpr int kPerSlot = (kReads + kMfmas - 1) / kMfmas;
+  auto interleave = [&](bool loads) {
 #pragma unroll
-    for (int g = 0; g < TM + TN; ++g) {
+    for (int g = 0; g < kMfmas; ++g) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    }
-#pragma unroll
-    for (int g = TM + TN; g < TM * TN; ++g) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-  };
-  auto interleave_loads = [&]() {
-#pragma unroll
-    for (int g = 0; g < TM * TN; ++g) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      if (g < TM + TN) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      if (g >= TM * TN - 2 * kLoads) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+      if (g * kPerSlot < kReads) __builtin_amdgcn_sched_group_barrier(0x100, kPerSlot, 0);
+      if (loads && kMfmas >= kPerStage && g >= kMfmas - kPerStage)
+        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
     }
   };
-  static_assert(TM * TN >= TM + TN && TM * TN >= 2 * kLoads, "MFMA slots for the reads and loads");
 
   // Every iteration loads one stage: past the last stage the loads repeat
   // it (in bounds, into a buffer no later stage uses), so the number of
@@ -654,17 +694,17 @@ GemmI8DmaKernel(const int8_t* __restrict__ QA, const float* __restrict__ sa,
     const int buf = it % kStages;
     read(buf, frag1, 1);
     mfmas(0);
-    interleave();
+    interleave(false);
     WaitVm<(kStages - 3) * kPerStage>();
     __builtin_amdgcn_s_barrier();
     issue(min(it + kStages - 1, last), (it + kStages - 1) % kStages);
     read((it + 1) % kStages, frag0, 0);
     mfmas(1);
-    interleave_loads();
+    interleave(true);
   }
   read(last % kStages, frag1, 1);
   mfmas(0);
-  interleave();
+  interleave(false);
   mfmas(1);
   WaitVm<0>();  // the repeated loads have landed before the workgroup ends
 
@@ -675,127 +715,64 @@ GemmI8DmaKernel(const int8_t* __restrict__ QA, const float* __restrict__ sa,
   const bool vec_out = (N % 4) == 0 && ((reinterpret_cast<uintptr_t>(C) |
                                          reinterpret_cast<uintptr_t>(sw) |
                                          reinterpret_cast<uintptr_t>(acc_out)) & 15) == 0;
+  auto store = [&](int m, int n, float s_a, int a0, int a1, int a2, int a3) {
+    const size_t at = static_cast<size_t>(m) * N + n;
+    if (vec_out && n + 3 < N) {
+      const float4 s4 = *reinterpret_cast<const float4*>(sw + n);
+      *reinterpret_cast<float4*>(C + at) =
+          make_float4((static_cast<float>(a0) * s_a) * s4.x, (static_cast<float>(a1) * s_a) * s4.y,
+                      (static_cast<float>(a2) * s_a) * s4.z, (static_cast<float>(a3) * s_a) * s4.w);
+      if (acc_out) *reinterpret_cast<int4*>(acc_out + at) = make_int4(a0, a1, a2, a3);
+    } else {
+      const int a[4] = {a0, a1, a2, a3};
 #pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int m = m0 + wm + i * 32 + lr;
-    if (m >= M) continue;
-    const float s_a = sa[m];
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int n = n0 + wn + j * 32 + 8 * q + 4 * h;
-        const size_t at = static_cast<size_t>(m) * N + n;
-        const v16i& a = acc[i][j];
-        if (vec_out && n + 3 < N) {
-          const float4 s4 = *reinterpret_cast<const float4*>(sw + n);
-          *reinterpret_cast<float4*>(C + at) =
-              make_float4((static_cast<float>(a[4 * q]) * s_a) * s4.x,
-                          (static_cast<float>(a[4 * q + 1]) * s_a) * s4.y,
-                          (static_cast<float>(a[4 * q + 2]) * s_a) * s4.z,
-                          (static_cast<float>(a[4 * q + 3]) * s_a) * s4.w);
-          if (acc_out)
-            *reinterpret_cast<int4*>(acc_out + at) =
-                make_int4(a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]);
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            if (n + e >= N) continue;
-            C[at + e] = (static_cast<float>(a[4 * q + e]) * s_a) * sw[n + e];
-            if (acc_out) acc_out[at + e] = a[4 * q + e];
-          }
-        }
+      for (int e = 0; e < 4; ++e) {
+        if (n + e >= N) continue;
+        C[at + e] = (static_cast<float>(a[e]) * s_a) * sw[n + e];
+        if (acc_out) acc_out[at + e] = a[e];
       }
-  }
-}
-
-// --- the small-M GEMM (decode-like) ---------------------------------------------
-
-// A workgroup per 16 kNT output columns; its kW waves each reduce one
-// contiguous K / kW slice (a 16-wave workgroup keeps 64 KB of the weight
-// stream in flight per CU), each activation fragment serving kNT weight
-// tiles; the int32 partials add exactly in any order.
-template <int MT, int kW, int kNT>  // M <= 16 MT rows; kW waves; 16 kNT columns
-__global__ void __launch_bounds__(kW * kWave)
-GemmI8SkinnyKernel(const int8_t* __restrict__ QA, const float* __restrict__ sa,
-                   const int8_t* __restrict__ QW, const float* __restrict__ sw,
-                   float* __restrict__ C, int32_t* __restrict__ acc_out, int M, int N, int K) {
-  constexpr int kTiles = MT * kNT;
-  static_assert(kTiles <= kW, "a reducing wave per tile");
-  __shared__ v4i part[kW][kTiles][kWave];
-  const int tid = threadIdx.x;
-  const int wave = tid / kWave, lane = tid % kWave;
-  const int n0 = blockIdx.x * 16 * kNT;
-  const int kq = K / kW;  // each wave reduces one contiguous slice of K
-  const int kb = wave * kq, ke = kb + kq;
-  const int kl = (lane / 16) * 16;
-  const int8_t* wrow[kNT];
+    }
+  };
+  if constexpr (KG == 1) {
 #pragma unroll
-  for (int c = 0; c < kNT; ++c) {
-    const int col = n0 + c * 16 + lane % 16;
-    wrow[c] = QW + static_cast<size_t>(col < N ? col : 0) * K;
-  }
-  v4i acc[MT][kNT];
+    for (int i = 0; i < TM; ++i) {
+      const int m = m0 + wm + i * 32 + lr;
+      if (m >= M) continue;
+      const float s_a = sa[m];
 #pragma unroll
-  for (int t = 0; t < MT; ++t)
+      for (int j = 0; j < TN; ++j)
 #pragma unroll
-    for (int c = 0; c < kNT; ++c) acc[t][c] = v4i{0, 0, 0, 0};
-#pragma unroll 4
-  for (int k = kb; k < ke; k += 64) {
-    v4i b[kNT];
+        for (int q = 0; q < 4; ++q)
+          store(m, n0 + wn + j * 32 + 8 * q + 4 * h, s_a, acc[i][j][4 * q], acc[i][j][4 * q + 1],
+                acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+    }
+  } else {
+    // The k-groups' partials meet in LDS (the stages are done with): every
+    // wave leaves its quads, then sums and stores one KG-th of its block's.
+    constexpr int kQuads = TM * TN * 4;
+    static_assert(KG * kWaves * kQuads * kWave * 16 <= KG * kStages * kStage, "partials fit");
+    static_assert(kQuads % KG == 0, "whole quads per group");
+    __syncthreads();
+    v4i* part = reinterpret_cast<v4i*>(smem_all);
 #pragma unroll
-    for (int c = 0; c < kNT; ++c)
-      b[c] = n0 + c * 16 + lane % 16 < N ? *reinterpret_cast<const v4i*>(wrow[c] + k + kl)
-                                         : v4i{0, 0, 0, 0};
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int t = 0; t < MT; ++t) {
-      const int m = t * 16 + lane % 16;
-      const v4i a = m < M ? *reinterpret_cast<const v4i*>(QA + static_cast<size_t>(m) * K + k + kl)
-                          : v4i{0, 0, 0, 0};
+      for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int c = 0; c < kNT; ++c)
-        acc[t][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b[c], acc[t][c], 0, 0, 0);
+        for (int q = 0; q < 4; ++q)
+          part[((kg * kWaves + wave) * kQuads + (i * TN + j) * 4 + q) * kWave + lane] =
+              v4i{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < kQuads / KG; ++e) {
+      const int x = kg * (kQuads / KG) + e, q = x % 4, j = x / 4 % TN, i = x / 4 / TN;
+      v4i sum = part[(wave * kQuads + x) * kWave + lane];
+#pragma unroll
+      for (int w = 1; w < KG; ++w) sum += part[((w * kWaves + wave) * kQuads + x) * kWave + lane];
+      const int m = m0 + wm + i * 32 + lr;
+      if (m < M) store(m, n0 + wn + j * 32 + 8 * q + 4 * h, sa[m], sum[0], sum[1], sum[2], sum[3]);
     }
   }
-#pragma unroll
-  for (int t = 0; t < MT; ++t)
-#pragma unroll
-    for (int c = 0; c < kNT; ++c) part[wave][t * kNT + c][lane] = acc[t][c];
-  __syncthreads();
-  if (wave >= kTiles) return;
-  // Wave w sums tile w over the K slices (integers: exact in any order).
-  const int t = wave / kNT, c = wave % kNT;
-  v4i sum = part[0][wave][lane];
-#pragma unroll
-  for (int w = 1; w < kW; ++w) sum += part[w][wave][lane];
-  const int col = n0 + c * 16 + lane % 16;
-  if (col >= N) return;
-  const float swn = sw[col];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int m = t * 16 + (lane / 16) * 4 + r;  // lane holds rows 4*(lane/16)+r
-    if (m >= M) continue;
-    const size_t o = static_cast<size_t>(m) * N + col;
-    if (acc_out) acc_out[o] = sum[r];
-    C[o] = (static_cast<float>(sum[r]) * sa[m]) * swn;
-  }
-}
-
-// --- any shape: one lane per output, for K not a multiple of the vector ------
-
-__global__ void __launch_bounds__(kThreads)
-GemmI8NaiveKernel(const int8_t* __restrict__ QA, const float* __restrict__ sa,
-                  const int8_t* __restrict__ QW, const float* __restrict__ sw,
-                  float* __restrict__ C, int32_t* __restrict__ acc_out, size_t M, size_t N,
-                  size_t K) {
-  const size_t i = static_cast<size_t>(blockIdx.x) * kThreads + threadIdx.x;
-  if (i >= M * N) return;
-  const size_t m = i / N, n = i % N;
-  int32_t s = 0;
-  for (size_t k = 0; k < K; ++k)
-    s += static_cast<int32_t>(QA[m * K + k]) * static_cast<int32_t>(QW[n * K + k]);
-  if (acc_out) acc_out[i] = s;
-  C[i] = (static_cast<float>(s) * sa[m]) * sw[n];
 }
 
 inline bool Aligned(const void* p, uintptr_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
@@ -813,6 +790,46 @@ int DeviceCUs() {
   cached[dev].store(n, std::memory_order_relaxed);
   return n;
 }
+
+namespace {
+
+enum class Tile { k32, k64Split, k64, k128, k256x128, k256 };
+
+// The direct-to-LDS tile for an M x N output: the one whose measured time at
+// its number of tiles per CU (x) is least.  A tile's time grows with K alike
+// for all of them, so K stays out.  Measured at K = 4096, us, MI355X:
+//
+//   tile (k-groups)    x <= 1               past that
+//   32 x 32 (4)        7.2                  11.2 at 2, 21.6 at 4
+//   64 x 64 (2)        10.9 at 1/2, 13.2    22.6 at 2, 40.7 at 4
+//   64 x 64 (1)        14.5 at 1/2, 15.9    19.3 at 2, 43 at 4, 81 at 8
+//   128 x 128          22 at 1/2, 28        50.7 at 2, 71 at 3, 93 at 4
+//   256 x 128          33 at 1/2, 45        74 at 1.5, 86.6 at 2
+//   256 x 256          47 at 1/4, 50 at 1/2, 59.6 at 3/4, 73 at 1
+//
+// The two largest run one workgroup per CU, so they pay by whole rounds of
+// the CUs.  Register-staged tiles of 128 x 128 ran all of these
+// before: 30-36 us for M from 65 to 1024 at 4096 x 4096, now 11-28.
+Tile PickTile(size_t M, size_t N) {
+  const double cus = DeviceCUs();
+  const auto x = [&](size_t bm, size_t bn) {
+    return static_cast<double>((M + bm - 1) / bm) * static_cast<double>((N + bn - 1) / bn) / cus;
+  };
+  const auto rounds = [](double v, double whole, double first, double slope) {
+    const double full = std::floor(v), part = v - full;
+    return whole * full + (part > 0 ? first + slope * part : 0.0);
+  };
+  const double x32 = x(32, 32), x64 = x(64, 64), x128 = x(128, 128);
+  const double t[] = {std::max(7.2, 6.0 * x32),
+                      std::max(9.5 + 3.7 * x64, 11.0 * x64),
+                      std::max(14.0 + 2.7 * x64, 10.2 * x64),
+                      std::max(17.0 + 11.0 * x128, 23.5 * x128),
+                      rounds(x(256, 128), 43.0, 20.0, 25.0),
+                      rounds(x(256, 256), 73.0, 25.0, 48.0)};
+  return static_cast<Tile>(std::min_element(t, t + 6) - t);
+}
+
+}  // namespace
 
 hipError_t LaunchQuantizeRows(const float* X, int8_t* Q, float* scale, size_t rows, size_t cols,
                               int waves_per_cu, hipStream_t s) {
@@ -867,55 +884,80 @@ hipError_t LaunchGemmW8A8(const int8_t* QA, const float* sa, const int8_t* QWt, 
                           float* C, int32_t* acc, size_t M, size_t N, size_t K,
                           const TilePolicy& policy, hipStream_t s) {
   if (M == 0 || N == 0) return hipSuccess;
-  const bool vec_ok = K % 16 == 0 && Aligned(QA, 16) && Aligned(QWt, 16) && M < (1u << 30) &&
-                      N < (1u << 30) && K < (1u << 30) && M * K < (1ull << 31) &&
-                      N * K < (1ull << 31);
-  if (vec_ok && M <= 64 && K % 256 == 0) {
-    const int m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);
-    const auto grid = [&](int cols) { return dim3(static_cast<unsigned>((N + cols - 1) / cols)); };
-    if (K % (64 * 16) == 0) {  // 16 waves of 64-deep steps (two column tiles per
-                               // fragment measured slower at 32 x 4096 x 4096)
-      if (M <= 32)
-        hipLaunchKernelGGL((GemmI8SkinnyKernel<2, 16, 1>), grid(16), dim3(16 * kWave), 0, s, QA, sa,
-                           QWt, sw, C, acc, m, n, k);
-      else
-        hipLaunchKernelGGL((GemmI8SkinnyKernel<4, 16, 1>), grid(16), dim3(16 * kWave), 0, s, QA, sa,
-                           QWt, sw, C, acc, m, n, k);
-    } else if (M <= 32) {
-      hipLaunchKernelGGL((GemmI8SkinnyKernel<2, 4, 1>), grid(16), dim3(4 * kWave), 0, s, QA, sa, QWt,
-                         sw, C, acc, m, n, k);
-    } else {
-      hipLaunchKernelGGL((GemmI8SkinnyKernel<4, 4, 1>), grid(16), dim3(4 * kWave), 0, s, QA, sa, QWt,
-                         sw, C, acc, m, n, k);
-    }
-    return hipGetLastError();
+  const bool dma = K > 0 && K % 16 == 0 && Aligned(QA, 16) && Aligned(QWt, 16) &&
+                   M < (1u << 30) && N < (1u << 30) && K * 256 < (1ull << 31) &&
+                   M * K < (1ull << 31) && N * K < (1ull << 31);
+  if (!dma) {
+    // Any K and alignment, in blocks whose indices fit 32 bits.  64 x 64 tiles
+    // up to three per CU, 128 x 128 of eight waves past that: 1024 x 4096 x
+    // 4095 68 / 56 us, 512 x 4096 x 4095 39 / 48 us, 1000 x 3000 x 999 18.2 /
+    // 18.5 us (one lane per output, as before: 11.5 ms).
+    constexpr size_t kMost = size_t{1} << 30;
+    for (size_t m0 = 0; m0 < M; m0 += kMost)
+      for (size_t n0 = 0; n0 < N; n0 += kMost) {
+        const size_t m = std::min(M - m0, kMost), n = std::min(N - n0, kMost);
+        const auto tiles = [&](size_t b) { return (m + b - 1) / b * ((n + b - 1) / b); };
+        const bool large = tiles(64) > 3 * static_cast<size_t>(DeviceCUs());
+        if (tiles(large ? 128 : 64) >= (size_t{1} << 31)) return hipErrorInvalidValue;
+        const size_t at = m0 * N + n0;
+        if (large)
+          hipLaunchKernelGGL((GemmI8TileKernel<128, 128, 128, 2, 4, false>),
+                             dim3(static_cast<unsigned>(tiles(128))), dim3(512), 0, s, QA + m0 * K,
+                             sa + m0, QWt + n0 * K, sw + n0, C + at, acc ? acc + at : nullptr,
+                             static_cast<int>(m), static_cast<int>(n), static_cast<int64_t>(K), N);
+        else
+          hipLaunchKernelGGL((GemmI8TileKernel<64, 64, 128, 2, 2, false>),
+                             dim3(static_cast<unsigned>(tiles(64))), dim3(256), 0, s, QA + m0 * K,
+                             sa + m0, QWt + n0 * K, sw + n0, C + at, acc ? acc + at : nullptr,
+                             static_cast<int>(m), static_cast<int>(n), static_cast<int64_t>(K), N);
+        if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+      }
+    return hipSuccess;
   }
-  if (vec_ok) {
-    // Tile geometry (TilePolicy): from M, N >= w8a8_large_min the policy's
-    // large kernel -- by default the direct-to-LDS 256 x 256 when K is a
-    // multiple of its 64-byte stage -- else 128 x 128 (four waves).
-    const bool big = M >= policy.w8a8_large_min && N >= policy.w8a8_large_min;
-    const int pick = !big ? 3 : policy.w8a8_large_kernel;
-    const bool dma_ok = K >= kDmaBK && K % kDmaBK == 0 && K * 256 < (1ull << 31);
-    if (pick == 1 && dma_ok) {
-      const unsigned tiles = static_cast<unsigned>(((M + 255) / 256) * ((N + 255) / 256));
-      hipLaunchKernelGGL((GemmI8DmaKernel<4, 2, 4>), dim3(tiles), dim3(512), 0, s, QA, sa, QWt, sw, C,
-                         acc, static_cast<int>(M), static_cast<int>(N), static_cast<int>(K));
-    } else if (pick <= 2) {
-      const unsigned tiles = static_cast<unsigned>(((M + 255) / 256) * ((N + 255) / 256));
-      hipLaunchKernelGGL((GemmI8TileKernel<256, 256, 128, 4, 4>), dim3(tiles), dim3(1024), 0, s, QA,
-                         sa, QWt, sw, C, acc, static_cast<int>(M), static_cast<int>(N),
-                         static_cast<int>(K));
-    } else {
-      const unsigned tiles = static_cast<unsigned>(((M + 127) / 128) * ((N + 127) / 128));
-      hipLaunchKernelGGL((GemmI8TileKernel<128, 128, 128, 2, 2>), dim3(tiles), dim3(256), 0, s, QA,
-                         sa, QWt, sw, C, acc, static_cast<int>(M), static_cast<int>(N),
-                         static_cast<int>(K));
+  const int m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);
+  const auto tiles = [&](size_t bm, size_t bn) {
+    return dim3(static_cast<unsigned>(((M + bm - 1) / bm) * ((N + bn - 1) / bn)));
+  };
+  // Tile geometry (TilePolicy): from M, N >= w8a8_large_min the policy's
+  // large kernel -- by default the direct-to-LDS 256 x 256.
+  const bool big = M >= policy.w8a8_large_min && N >= policy.w8a8_large_min;
+  if (big && policy.w8a8_large_kernel == 2)
+    hipLaunchKernelGGL((GemmI8TileKernel<256, 256, 128, 4, 4, true>), tiles(256, 256), dim3(1024), 0,
+                       s, QA, sa, QWt, sw, C, acc, m, n, static_cast<int64_t>(k), N);
+  else if (big && policy.w8a8_large_kernel >= 3)
+    hipLaunchKernelGGL((GemmI8TileKernel<128, 128, 128, 2, 2, true>), tiles(128, 128), dim3(256), 0,
+                       s, QA, sa, QWt, sw, C, acc, m, n, static_cast<int64_t>(k), N);
+  else
+    switch (big ? Tile::k256 : PickTile(M, N)) {
+      case Tile::k32:
+        hipLaunchKernelGGL((GemmI8DmaKernel<32, 32, 6, 1, 1, 4>), tiles(32, 32), dim3(256), 0, s, QA,
+                           sa, QWt, sw, C, acc, m, n, k);
+        break;
+      case Tile::k64Split:
+        hipLaunchKernelGGL((GemmI8DmaKernel<64, 64, 4, 2, 2, 2>), tiles(64, 64), dim3(512), 0, s, QA,
+                           sa, QWt, sw, C, acc, m, n, k);
+        break;
+      case Tile::k64:
+        hipLaunchKernelGGL((GemmI8DmaKernel<64, 64, 4, 2, 2, 1>), tiles(64, 64), dim3(256), 0, s, QA,
+                           sa, QWt, sw, C, acc, m, n, k);
+        break;
+      case Tile::k128:
+        hipLaunchKernelGGL((GemmI8DmaKernel<128, 128, 4, 2, 2, 1>), tiles(128, 128), dim3(256), 0, s,
+                           QA, sa, QWt, sw, C, acc, m, n, k);
+        break;
+      case Tile::k256x128:
+        hipLaunchKernelGGL((GemmI8DmaKernel<256, 128, 4, 4, 2, 1>), tiles(256, 128), dim3(512), 0, s,
+                           QA, sa, QWt, sw, C, acc, m, n, k);
+        break;
+      case Tile::k256:
+        if (K % kDmaBK == 0)
+          hipLaunchKernelGGL((GemmI8DmaKernel<256, 256, 4, 2, 4, 1, false>), tiles(256, 256),
+                             dim3(512), 0, s, QA, sa, QWt, sw, C, acc, m, n, k);
+        else
+          hipLaunchKernelGGL((GemmI8DmaKernel<256, 256, 4, 2, 4, 1>), tiles(256, 256), dim3(512), 0,
+                             s, QA, sa, QWt, sw, C, acc, m, n, k);
+        break;
     }
-    return hipGetLastError();
-  }
-  hipLaunchKernelGGL(GemmI8NaiveKernel, dim3(GridFor(M * N, kThreads, 1u << 30)), dim3(kThreads), 0,
-                     s, QA, sa, QWt, sw, C, acc, M, N, K);
   return hipGetLastError();
 }
 

@@ -1876,6 +1876,42 @@ def test_w8a8_at_the_bench_shapes(hip, orc, torch_cuda, M):
     ctx.close()
 
 
+# Per direct-to-LDS tile (32, 64 with two k-groups, 64, 128, 256 x 128, 256): rows
+# and columns off the tile, K off the 64-byte stage; then any K and alignment
+# (64 and 128 tiles), down to one element.
+@pytest.mark.parametrize("M,N,K,shift", [
+    (1, 33, 16, 0), (63, 4095, 80, 0), (130, 4000, 1008, 0), (511, 4098, 144, 0),
+    (500, 5632, 272, 0), (2047, 4094, 48, 0), (3000, 4001, 336, 0), (3000, 4001, 320, 0),
+    (1, 1, 1, 0), (65, 63, 127, 0), (70, 66, 129, 0), (40, 130, 64, 3), (1500, 3002, 131, 0)])
+def test_w8a8_tiles_and_ragged_rows(hip, torch_cuda, M, N, K, shift):
+    """The int32 accumulators against an exact float64 product and C against
+    its own expression, bit for bit; `shift` starts both operands that many
+    bytes past a 16-byte boundary."""
+    torch = torch_cuda
+    print(f"w8a8 tile M={M} N={N} K={K} shift={shift}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+
+    def operand(rows):
+        flat = torch.randint(-127, 128, (rows * K + shift,), dtype=torch.int8, device="cuda",
+                             generator=g)
+        return flat[shift:].view(rows, K)
+    QA, QWt = operand(M), operand(N)
+    sa, sw = (torch.rand(n, device="cuda", generator=g) for n in (M, N))
+    C = torch.full((M, N), float("nan"), device="cuda")
+    acc = torch.full((M, N), -7, dtype=torch.int32, device="cuda")
+    ctx = hip.Context(0)
+    ctx.use_torch_stream()
+    for with_acc in (True, False):
+        ctx.call("seeai_w8a8_gemm", QA.data_ptr(), sa.data_ptr(), QWt.data_ptr(), sw.data_ptr(),
+                 C.data_ptr(), acc.data_ptr() if with_acc else None, M, N, K)
+        torch.cuda.synchronize()
+        want = (QA.double() @ QWt.double().t()).to(torch.int32)
+        assert torch.equal(acc, want), "int32 accumulators"
+        assert torch.equal(C, (want.float() * sa[:, None]) * sw[None]), "dequantized output"
+        C.fill_(float("nan"))
+    ctx.close()
+
+
 @pytest.mark.parametrize("cols", [1024, 2052, 4096, 4100])
 def test_w8a8_quantizer_on_half_level_quotients(hip, orc, torch_cuda, cols):
     """Every element's quotient x / scale sits within a few ulps of a half
