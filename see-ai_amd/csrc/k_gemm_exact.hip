@@ -17,9 +17,11 @@
 // sums are separate IEEE operations (no contraction: -ffp-contract=off and
 // __fmul_rn / __fadd_rn).
 //
-// Three shapes of kernel share these chains: short K (the whole panel in
-// LDS, one output per lane), long K over few outputs (quads formed in
-// parallel, folded in order), and the general tiled kernel.
+// Several shapes of kernel share these chains: short K over few outputs (the
+// whole panel in LDS, one output per lane), long K over few outputs (quads
+// formed in parallel, folded in order), rows of a middling number of outputs
+// (A through the scalar cache), 32 x 32 one-wave tiles for more, and the
+// general tiled kernel.
 //
 // Tiled: a BM x BN tile of C per 256-lane workgroup, each lane a TM x TN
 // register block, K walked in steps of 16 through LDS (k-major: As[k][m],
@@ -27,7 +29,6 @@
 // current one accumulates.  Every output has one writer.  The chains are
 // VALU multiply-adds (two operations per product), which bounds the kernel
 // at half the non-packed f32 VALU rate.
-#include <cstdlib>
 
 #include "common.h"
 
@@ -234,6 +235,202 @@ __global__ void __launch_bounds__(kThreads) GemmExactKernel(GemmArgs g) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// The NN / TN chains over up to a thousand or so 64 x 64 blocks of outputs
+// (TileFits; past that GemmExactKernel is as fast or faster): a 32 x 32 tile
+// per one-wave workgroup, 4 x 4 outputs a lane, so 2048 x 768 outputs are six
+// waves a CU rather than one and a half 64 x 64 workgroups.  The chains are
+// VALU work -- four multiplies and four adds a quad and output, no
+// contraction -- which the kernel reaches 85 % of the measured rate of (two
+// VALU operations a product: about 50 TFLOP/s) where the waves divide evenly.  K moves 16 at
+// a time through two LDS buffers (k-major), the next step's operands in
+// flight in registers as they were loaded: the scales apply at the LDS store,
+// so no load is waited for before the step's arithmetic.  Larger register
+// blocks (8 x 4, 8 x 8) leave one wave a SIMD and measured half as fast.
+// us: 2048 x 768 x 768 167 on the chain kernel, 95 on 64 x 64 tiles, 69 here;
+// 2048 x 768 x 3072 540 / 341 / 256; 4096 x 512 x 512 355 (panel) / 67 / 51.
+// ---------------------------------------------------------------------------
+constexpr int kTile = 32;
+
+template <int kLayout, int kBKind>
+__global__ void __launch_bounds__(kWave) GemmExactTileKernel(GemmArgs g, unsigned tiles_m) {
+  static_assert(kLayout != 1, "NN / TN");
+  constexpr int BM = kTile, BN = kTile, TM = 4, TN = 4;
+  constexpr int kT = kWave, kTX = BN / TN;
+  constexpr int kLdA = BM + 4, kLdB = BN + 4;
+  constexpr int kA = BM * kBK / 4 / kT, kB = BN * kBK / 4 / kT;  // float4 per lane and step
+  __shared__ __attribute__((aligned(16))) float As[2][kBK * kLdA];
+  __shared__ __attribute__((aligned(16))) float Bs[2][kBK * kLdB];
+  const int tid = threadIdx.x, tx = tid % kTX, ty = tid / kTX;
+  // Workgroups are dealt to the eight XCDs round-robin: XCD x takes a run of
+  // consecutive tiles, rows fastest, so B's columns are read through one L2.
+  const unsigned nt = gridDim.x, x = blockIdx.x % 8, rest = nt % 8;
+  const unsigned tile = x * (nt / 8) + min(x, rest) + blockIdx.x / 8;
+  const size_t m0 = static_cast<size_t>(tile % tiles_m) * BM;
+  const size_t n0 = static_cast<size_t>(tile / tiles_m) * BN;
+  const size_t M = g.M, N = g.N, K = g.K;
+
+  const auto row = [&](int i) { return TM * ty + i; };
+  const auto col = [&](int j) { return TN * tx + j; };
+
+  float acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = 0.0f;
+  if (g.accumulate) {  // GemmAccNN: the chains start at C
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const size_t m = m0 + row(i), n = n0 + col(j);
+        if (m < M && n < N) acc[i][j] = g.C[m * N + n];
+      }
+  }
+
+  // This lane's loads of a step.  Rows (columns) past the end repeat the
+  // last whole group: their outputs are not stored.  k past the end repeats
+  // the last k: not used.
+  float4 ra[kA], rs[kA];
+  float4 rb[kB];
+  uint32_t rq[kB];
+  uint2 rh[kB];
+  auto load = [&](size_t k0) {
+#pragma unroll
+    for (int e = 0; e < kA; ++e) {
+      const int idx = tid + e * kT;
+      if constexpr (kLayout == 2) {  // A[K, M]: m fastest
+        const size_t m = min(m0 + idx % (BM / 4) * 4, M - 4), k = min(k0 + idx / (BM / 4), K - 1);
+        ra[e] = *reinterpret_cast<const float4*>(g.A + k * M + m);
+      } else {                       // A[M, K]: k fastest
+        const size_t m = min(m0 + idx / 4, M - 1), k = min(k0 + idx % 4 * 4, K - 4);
+        ra[e] = *reinterpret_cast<const float4*>(g.A + m * K + k);
+        if (g.a_k_scale) rs[e] = *reinterpret_cast<const float4*>(g.a_k_scale + k);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < kB; ++e) {
+      const int idx = tid + e * kT;
+      const size_t n = min(n0 + idx % (BN / 4) * 4, N - 4), k = min(k0 + idx / (BN / 4), K - 1);
+      if constexpr (kBKind == 0)
+        rb[e] = *reinterpret_cast<const float4*>(static_cast<const float*>(g.B) + k * N + n);
+      else if constexpr (kBKind == 1)
+        rq[e] = *reinterpret_cast<const uint32_t*>(static_cast<const int8_t*>(g.B) + k * N + n);
+      else
+        rh[e] = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(g.B) + k * N + n);
+    }
+  };
+  float4 bscale[kBKind == 1 ? kB : 1];
+  if constexpr (kBKind == 1) {
+    if (g.b_col_scale) {
+#pragma unroll
+      for (int e = 0; e < kB; ++e) {
+        const float* p = g.b_col_scale + min(n0 + (tid + e * kT) % (BN / 4) * 4, N - 4);
+        bscale[e] = make_float4(p[0], p[1], p[2], p[3]);
+      }
+    }
+  }
+  auto store = [&](int buf) {
+#pragma unroll
+    for (int e = 0; e < kA; ++e) {
+      const int idx = tid + e * kT;
+      float4 v = ra[e];
+      if (kLayout != 2 && g.a_k_scale)
+        v = make_float4(Mul(v.x, rs[e].x), Mul(v.y, rs[e].y), Mul(v.z, rs[e].z), Mul(v.w, rs[e].w));
+      if (g.alpha_a != 1.0f)
+        v = make_float4(Mul(g.alpha_a, v.x), Mul(g.alpha_a, v.y), Mul(g.alpha_a, v.z),
+                        Mul(g.alpha_a, v.w));
+      if constexpr (kLayout == 2) {
+        *reinterpret_cast<float4*>(&As[buf][idx / (BM / 4) * kLdA + idx % (BM / 4) * 4]) = v;
+      } else {
+        float* a = &As[buf][idx % 4 * 4 * kLdA + idx / 4];
+        a[0] = v.x, a[kLdA] = v.y, a[2 * kLdA] = v.z, a[3 * kLdA] = v.w;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < kB; ++e) {
+      const int idx = tid + e * kT;
+      float4 v;
+      if constexpr (kBKind == 0) {
+        v = rb[e];
+      } else if constexpr (kBKind == 1) {
+        const auto w = [&](int u) { return static_cast<float>(static_cast<int8_t>(rq[e] >> (8 * u))); };
+        v = make_float4(w(0), w(1), w(2), w(3));
+        if (g.b_col_scale)
+          v = make_float4(Mul(v.x, bscale[e].x), Mul(v.y, bscale[e].y), Mul(v.z, bscale[e].z),
+                          Mul(v.w, bscale[e].w));
+      } else {
+        v = make_float4(Bf16ToF32(rh[e].x & 0xffff), Bf16ToF32(rh[e].x >> 16),
+                        Bf16ToF32(rh[e].y & 0xffff), Bf16ToF32(rh[e].y >> 16));
+      }
+      *reinterpret_cast<float4*>(&Bs[buf][idx / (BN / 4) * kLdB + idx % (BN / 4) * 4]) = v;
+    }
+  };
+  auto frag = [&](int buf, int k, float* a, float* b) {
+    const float4 u = *reinterpret_cast<const float4*>(&As[buf][k * kLdA + row(0)]);
+    const float4 v = *reinterpret_cast<const float4*>(&Bs[buf][k * kLdB + col(0)]);
+    a[0] = u.x, a[1] = u.y, a[2] = u.z, a[3] = u.w;
+    b[0] = v.x, b[1] = v.y, b[2] = v.z, b[3] = v.w;
+  };
+  auto quad = [&](int buf, int kk) {
+    float a0[TM], a1[TM], a2[TM], a3[TM], b0[TN], b1[TN], b2[TN], b3[TN];
+    frag(buf, kk + 0, a0, b0);
+    frag(buf, kk + 1, a1, b1);
+    frag(buf, kk + 2, a2, b2);
+    frag(buf, kk + 3, a3, b3);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const float q = Add(Add(Add(Mul(a0[i], b0[j]), Mul(a1[i], b1[j])), Mul(a2[i], b2[j])),
+                            Mul(a3[i], b3[j]));
+        acc[i][j] = Add(acc[i][j], q);
+      }
+  };
+
+  load(0);
+  store(0);
+  __syncthreads();
+  int buf = 0;
+  size_t k0 = 0;
+  for (; k0 + kBK < K; k0 += kBK) {
+    load(k0 + kBK);
+#pragma unroll
+    for (int kk = 0; kk < kBK; kk += 4) quad(buf, kk);
+    store(buf ^ 1);
+    __syncthreads();
+    buf ^= 1;
+  }
+  const int kn = static_cast<int>(K - k0), kq = kn & ~3;
+  for (int kk = 0; kk < kq; kk += 4) quad(buf, kk);
+  for (int kk = kq; kk < kn; ++kk) {  // the K % 4 tail, one term at a time
+    float a[TM], b[TN];
+    frag(buf, kk, a, b);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = Add(acc[i][j], Mul(a[i], b[j]));
+  }
+
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const size_t m = m0 + row(i);
+    const size_t n = n0 + col(0);
+    if (m >= M || n >= N) continue;  // N % 4 == 0: whole groups
+    float c[4] = {acc[i][0], acc[i][1], acc[i][2], acc[i][3]};
+    if (g.addend) {
+      const float4 d = *reinterpret_cast<const float4*>(g.addend + m * N + n);
+      c[0] = Add(d.x, c[0]), c[1] = Add(d.y, c[1]), c[2] = Add(d.z, c[2]), c[3] = Add(d.w, c[3]);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (g.bias) c[e] = Add(c[e], g.bias[n + e]);
+      if (g.act) c[e] = ActExpr(g.act, c[e]);
+    }
+    *reinterpret_cast<float4*>(g.C + m * N + n) = make_float4(c[0], c[1], c[2], c[3]);
+  }
+}
+
 // Staged A element (m, k): the q8 k-scale and the NN / TN alpha applied as
 // the reference applies them, one rounding each.
 template <int kLayout>
@@ -250,6 +447,87 @@ __device__ __forceinline__ float Epilogue(const GemmArgs& g, size_t m, size_t n,
   if (g.bias) c = Add(c, g.bias[n]);
   if (g.act) c = ActExpr(g.act, c);
   return c;
+}
+
+// ---------------------------------------------------------------------------
+// NN over a middling number of outputs (RowsFits): the LDS tiles above would
+// leave most SIMDs one wave or none, and a lone wave is bound by its own
+// latency.  A wave owns kRowsM rows x 64 columns, a column per lane: A's
+// quads are wave-uniform and come through the scalar cache straight into the
+// multiplies, B's through four quads of coalesced loads in flight -- no LDS,
+// no barrier, four waves a workgroup on neighbouring rows of the same columns.
+// ---------------------------------------------------------------------------
+constexpr int kRowsM = 2, kRowsWaves = kThreads / kWave;
+
+template <int kBKind>
+__global__ void __launch_bounds__(kThreads, 4)
+GemmExactRowsKernel(GemmArgs g, const float* __restrict__ A, const void* __restrict__ B,
+                    unsigned tiles_m) {
+  const int lane = threadIdx.x % kWave, wave = Uniform(threadIdx.x / kWave);
+  // XCD x takes a run of consecutive tiles, rows fastest.
+  const unsigned nt = gridDim.x, x = blockIdx.x % 8, rest = nt % 8;
+  const unsigned tile = x * (nt / 8) + min(x, rest) + blockIdx.x / 8;
+  const size_t M = g.M, N = g.N, K = g.K;
+  const size_t m0 = (static_cast<size_t>(tile % tiles_m) * kRowsWaves + wave) * kRowsM;
+  const size_t n = static_cast<size_t>(tile / tiles_m) * kWave + lane, nl = min(n, N - 1);
+  if (m0 >= M) return;  // wave-uniform; no barrier follows
+  const float* arow[kRowsM];
+#pragma unroll
+  for (int i = 0; i < kRowsM; ++i) arow[i] = A + min(m0 + i, M - 1) * K;
+  struct Quad { float v[4]; };
+  const auto load_b = [&](size_t k, Quad& b) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      b.v[u] = LoadB<0, kBKind>(B, N, K, nl, k + u, g.b_col_scale);
+  };
+  const auto load_a = [&](size_t k, Quad (&a)[kRowsM]) {
+#pragma unroll
+    for (int i = 0; i < kRowsM; ++i)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) a[i].v[u] = arow[i][k + u];
+  };
+  float acc[kRowsM];
+#pragma unroll
+  for (int i = 0; i < kRowsM; ++i)
+    acc[i] = g.accumulate && m0 + i < M && n < N ? g.C[(m0 + i) * N + n] : 0.0f;
+  const auto quad = [&](const Quad (&a)[kRowsM], const Quad& b) {
+#pragma unroll
+    for (int i = 0; i < kRowsM; ++i)
+      acc[i] = Add(acc[i], Add(Add(Add(Mul(a[i].v[0], b.v[0]), Mul(a[i].v[1], b.v[1])),
+                                   Mul(a[i].v[2], b.v[2])), Mul(a[i].v[3], b.v[3])));
+  };
+  // Four quads of B and one of A ahead; past the last quad the loads repeat it.
+  Quad a0[kRowsM], a1[kRowsM], b0, b1, b2, b3;
+  const size_t last = K - 4;
+  load_a(0, a0);
+  load_b(0, b0);
+  load_b(min(size_t{4}, last), b1);
+  load_b(min(size_t{8}, last), b2);
+  load_b(min(size_t{12}, last), b3);
+  size_t k = 0;
+  for (; k + 16 <= K; k += 16) {
+    load_a(k + 4, a1);
+    quad(a0, b0);
+    load_b(min(k + 16, last), b0);
+    load_a(k + 8, a0);
+    quad(a1, b1);
+    load_b(min(k + 20, last), b1);
+    load_a(k + 12, a1);
+    quad(a0, b2);
+    load_b(min(k + 24, last), b2);
+    load_a(min(k + 16, last), a0);
+    quad(a1, b3);
+    load_b(min(k + 28, last), b3);
+  }
+  if (k < K) {  // one to three quads left (K % 4 == 0)
+    quad(a0, b0);
+    if (k + 4 < K) load_a(k + 4, a0), quad(a0, b1);
+    if (k + 8 < K) load_a(k + 8, a0), quad(a0, b2);
+  }
+  if (n >= N) return;
+#pragma unroll
+  for (int i = 0; i < kRowsM; ++i)
+    if (m0 + i < M) g.C[(m0 + i) * N + n] = Epilogue(g, m0 + i, n, acc[i]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1423,9 +1701,12 @@ hipError_t LaunchFold(const GemmArgs& a, hipStream_t s) {
 
 // The chain kernel where the tiled kernel's grid would be small for the
 // reduction it carries: under 512 tiles of 64 x 64 and K above the panel.
+// NT's tiled kernel (32 x 64 blocks, eight chains an output) takes over
+// earlier: 512 x 2560 x 704, 320 blocks of 64 x 64, 136 us here and 115 there;
+// 512 x 768 x 768, 96 blocks, 33 and 59.
 bool Chain(const GemmArgs& a) {
   const size_t tiles = ((a.M + 63) / 64) * ((a.N + 63) / 64);
-  return a.K > static_cast<size_t>(kPanelK) && tiles < 512;
+  return a.K > static_cast<size_t>(kPanelK) && tiles < (a.layout == 1 ? 320 : 512);
 }
 
 template <int kLayout, int kBKind, int BM, int BN>
@@ -1484,6 +1765,67 @@ hipError_t LaunchQuadsFold(const GemmArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+// What GemmExactTileKernel's 16-byte loads and stores assume.
+bool TileFits(const GemmArgs& a) {
+  const auto al = [](const void* p, uintptr_t n) { return reinterpret_cast<uintptr_t>(p) % n == 0; };
+  const uintptr_t b = a.b_kind == 0 ? 16 : a.b_kind == 1 ? 4 : 8;
+  return a.layout != 1 && a.N >= 4 && a.N % 4 == 0 && al(a.B, b) && al(a.A, 16) && al(a.C, 16) &&
+         al(a.addend, 16) && (a.layout == 2 ? a.M >= 4 && a.M % 4 == 0 && a.K > 0 && !a.a_k_scale
+                                            : a.K >= 4 && a.K % 4 == 0 && al(a.a_k_scale, 16));
+}
+
+size_t Tiles64(const GemmArgs& a) { return ((a.M + 63) / 64) * ((a.N + 63) / 64); }
+
+// Where the 32 x 32 tiles run: enough of them to give every SIMD its wave
+// (below, the rows kernel and the small-output routes are faster: 1024 x 512
+// x 512, 128 blocks of 64 x 64, 44 us against 27), and not so many that the
+// 64 x 64 tiles' lower LDS traffic counts (2048 x 32000 x 768: 2339 us
+// against 2096; 8192 x 768 x 768, 1536 blocks: 225 / 222).
+bool Tile(const GemmArgs& a) {
+  return TileFits(a) && a.M >= kTile && a.N >= kTile && Tiles64(a) >= 200 && Tiles64(a) < 1024;
+}
+
+template <int kLayout, int kBKind>
+hipError_t LaunchTile(const GemmArgs& a, hipStream_t s) {
+  const size_t tm = (a.M + kTile - 1) / kTile, tn = (a.N + kTile - 1) / kTile;
+  if (tm * tn >= (size_t{1} << 31)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((GemmExactTileKernel<kLayout, kBKind>), dim3(static_cast<unsigned>(tm * tn)),
+                     dim3(kWave), 0, s, a, static_cast<unsigned>(tm));
+  return hipGetLastError();
+}
+
+// Where the rows kernel runs (whole quads of unscaled A): below the tiles, or
+// too few rows for them.  us, old route / rows: 1024 x 512 x 512 74 (panel) /
+// 28, 1024 x 256 x 256 15 / 10.5, 2048 x 128 x 128 9.3 / 7.0, 512 x 768 x 768
+// 39 (chain) / 33, 8 x 32000 x 768 40 / 31; but 256 x 768 x 768 (48 blocks) 21
+// / 26, 64 x 256 x 256 (4) 8.8 / 9.3.
+bool Rows(const GemmArgs& a) {
+  if (a.layout != 0 || a.K < 4 || a.K % 4 != 0 || a.alpha_a != 1.0f || a.a_k_scale || a.N < 64)
+    return false;
+  const size_t t = Tiles64(a);
+  return t >= (a.K <= static_cast<size_t>(kPanelK) ? 32u : 80u) && (t < 200 || a.M < kTile);
+}
+
+template <int kBKind>
+hipError_t LaunchRows(const GemmArgs& a, hipStream_t s) {
+  const size_t tm = (a.M + kRowsM * kRowsWaves - 1) / (kRowsM * kRowsWaves);
+  const size_t tn = (a.N + kWave - 1) / kWave;
+  if (tm * tn >= (size_t{1} << 31)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((GemmExactRowsKernel<kBKind>), dim3(static_cast<unsigned>(tm * tn)),
+                     dim3(kThreads), 0, s, a, a.A, a.B, static_cast<unsigned>(tm));
+  return hipGetLastError();
+}
+
+// The panel kernel reads both operands from LDS for every product: past the
+// outputs that fill the machine with one lane each, the tiled kernel's
+// register blocks are several times faster (us, panel / tiled: 1024 x 512 x
+// 512 NT, 128 blocks of 64 x 64, 92 / 41; 8192 x 2048 x 512 NN 2760 / 390, NT
+// 3382 / 660; but 1024 x 256 x 256 NT, 64 blocks, 17 / 22).
+bool Panel(const GemmArgs& a) {
+  return a.K > 0 && a.K <= static_cast<size_t>(kPanelK) && (a.M + 15) / 16 <= 65535 &&
+         (a.M <= 16 || Tiles64(a) < 100);
+}
+
 template <int kLayout, int kBKind>
 hipError_t Run(const GemmArgs& a, hipStream_t s) {
   if (kBKind == 0 && RankFits(a)) {
@@ -1501,7 +1843,13 @@ hipError_t Run(const GemmArgs& a, hipStream_t s) {
       return hipGetLastError();
     }
   }
-  if (a.K <= static_cast<size_t>(kPanelK) && a.K > 0 && (a.M + 15) / 16 <= 65535) {
+  if constexpr (kLayout == 0)
+    if (Rows(a)) return LaunchRows<kBKind>(a, s);
+  if constexpr (kLayout != 1) {
+    const bool fold = Fold(a) || FoldNarrowNN(a) || (LongK(a) && a.scratch && LongKFirst(a));
+    if (Tile(a) && !fold) return LaunchTile<kLayout, kBKind>(a, s);
+  }
+  if (Panel(a)) {
     const dim3 grid(static_cast<unsigned>((a.N + 15) / 16), static_cast<unsigned>((a.M + 15) / 16));
     const size_t lds = 2 * 16 * a.K * sizeof(float);
     hipLaunchKernelGGL((GemmPanelKernel<kLayout, kBKind>), grid, dim3(kThreads), lds, s, a);

@@ -276,6 +276,23 @@ def test_gemm_narrow_weights(hip, orc, backend, M, N, K):
             assert bits_equal(g, c), f"{name} {M}x{N}x{K}: not bit-exact (max-rel {maxrel(g, c):.3g})"
 
 
+# The 32 x 32 one-wave tiles (200 to 1023 blocks of 64 x 64, whole float4
+# rows), the rows kernel (fewer, or few rows) and, past the panel kernel, the
+# general tiled kernel (rows off float4): off every tile, K off the 16-deep step.
+TILES_AND_ROWS = [(830, 1100, 68), (803, 1028, 44), (515, 260, 36), (5, 4100, 20),
+                  (640, 524, 524), (806, 1030, 67)]
+
+
+@pytest.mark.parametrize("M,N,K", TILES_AND_ROWS)
+def test_gemm_f32_on_tiles_and_rows(hip, orc, backend, M, N, K):
+    test_gemm_f32_family(hip, orc, backend, M, N, K, False)
+
+
+@pytest.mark.parametrize("M,N,K", TILES_AND_ROWS)
+def test_gemm_narrow_weights_on_tiles_and_rows(hip, orc, backend, M, N, K):
+    test_gemm_narrow_weights(hip, orc, backend, M, N, K)
+
+
 # --- elementwise / activation / normalization -------------------------------------
 
 def test_elementwise_family(hip, orc, backend):
