@@ -887,7 +887,8 @@ uint64_t CurIndex(const seeai_ctx* c) { return static_cast<uint64_t>(c->cur_at -
 // A relaxed product on the direct-to-LDS kernel whose C the softmax-xent
 // forward right after takes as its logits: its epilogue also leaves C's
 // partial row maxima (a->row_max_part), from which the loss turn forms the
-// row max without its own pass over the logits.
+// row max without its own pass over the logits -- for rows too long for the
+// turn to hold (XEntRowResident).
 int PlanRowMaxParts(seeai_ctx* c, GemmArgs* a) {
   if (!c->allow_fusion || !c->cur_at || !c->prog || !a->relaxed || !c->allow_dma) return SEEAI_OK;
   const uint64_t idx = CurIndex(c);
@@ -896,7 +897,7 @@ int PlanRowMaxParts(seeai_ctx* c, GemmArgs* a) {
   std::memcpy(&nx, c->prog + (idx + 1) * 64, sizeof nx);
   const Ptrs R{c};
   if ((nx.opcode != 11 && nx.opcode != 51) || R.f(nx.in[0]) != a->C || nx.out[0] != a->M ||
-      nx.out[1] != a->N || XEntOneWorkgroup(a->M, a->N))
+      nx.out[1] != a->N || XEntOneWorkgroup(a->M, a->N) || XEntRowResident(a->N))
     return SEEAI_OK;
   a->policy = &c->policy;
   if (!Bf16DmaRowMaxFits(*a) || !Immutable(c, a->B)) return SEEAI_OK;

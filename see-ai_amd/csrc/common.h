@@ -254,6 +254,9 @@ hipError_t LaunchXEntFwdBwd(const float* logits, const int32_t* labels, float* l
 // Whether the fused loss turn of N rows of C runs in one workgroup (no row
 // max pass).
 bool XEntOneWorkgroup(size_t N, size_t C);
+// Whether the turn holds whole rows of C in registers (longer rows run a row
+// max pass of their own).
+bool XEntRowResident(size_t C);
 // max_parts: the logits' partial row maxima [N, ceil(C / 64)] a GEMM
 // epilogue left (GemmArgs::row_max_part); the row max is formed from them.
 // Whether the backward's row kernel can feed a sink (float4 rows).

@@ -465,6 +465,61 @@ def test_xent_forward_fill_backward_fuse_bitwise(hip, orc, backend, masked, read
         assert e <= TOL, f"{name}: {e:.3g}"
 
 
+def _loss_rows(kind, C):
+    """Rows that steer the exp-sum chain: the sum's path through the binades,
+    ties on the grid, subnormal starts, infinities and NaN."""
+    r = rng(len(kind) * C)
+    x = (r.standard_normal((6, C)) * {"narrow": 0.1, "wide": 30.0}.get(kind, 3.0)).astype(np.float32)
+    if kind == "falling":
+        x = -np.sort(-x, axis=1)
+    elif kind == "rising":
+        x = np.sort(x * 20, axis=1)
+    elif kind == "ties":  # exp of -24 ln 2 is 2^-24: half a grid step at a sum of 1
+        x[:, :] = np.float32(-24 * np.log(2.0))
+        x[:, 0] = 0.0
+        x[1, C // 2] = 0.0
+        x[2:, ::7] = -5.0
+    elif kind == "subnormal":
+        x[:, : C // 2] = np.float32(-95.0) - r.random((6, C // 2)).astype(np.float32) * 12
+        x[:, -1] = 40.0
+    elif kind == "special":
+        x[0, :] = 2.5
+        x[1, 3 % C] = np.nan
+        x[2, 5 % C] = np.inf
+        x[3, ::2] = -np.inf
+        x[4, :] = -np.inf
+        x[5, :-1] = np.finfo(np.float32).min
+    return x
+
+
+@pytest.mark.parametrize("kind", ["plain", "narrow", "wide", "falling", "rising", "ties",
+                                  "subnormal", "special"])
+@pytest.mark.parametrize("C", [1, 255, 1024, 1025, 4099, 8192, 16001, 32000, 32768])
+def test_xent_rows_in_registers_keep_the_chain(hip, torch_cuda, C, kind):
+    """Rows of at most 32768 columns run one pass with the exp-sum chain in
+    parallel: every probability bit for bit expf(x - max) times the reciprocal
+    of those terms' serial f32 sum (numpy's running sum, in column order)."""
+    torch = torch_cuda
+    print(f"xent chain C={C} {kind}", flush=True)
+    x = torch.from_numpy(_loss_rows(kind, C)).cuda()
+    N = x.shape[0]
+    labels = torch.arange(N, dtype=torch.int32, device="cuda") * 3 % C
+    loss, probs = torch.full((1,), -1.0, device="cuda"), torch.full_like(x, -1.0)
+    ctx = hip.Context(0)
+    ctx.use_torch_stream()
+    ctx.call("seeai_xent_fwd", x.data_ptr(), labels.data_ptr(), loss.data_ptr(), probs.data_ptr(),
+             N, C, 0)
+    torch.cuda.synchronize()
+    mx = torch.from_numpy(np.fmax.reduce(x.cpu().numpy(), axis=1)).cuda()
+    e = torch.exp(x - mx[:, None]).cpu().numpy()  # the same device expf
+    with np.errstate(invalid="ignore"):
+        total = np.add.accumulate(e, axis=1, dtype=np.float32)[:, -1]
+        want = e * (np.float32(1.0) / total)[:, None]
+    got = probs.cpu().numpy()
+    assert np.array_equal(got, want, equal_nan=True), np.flatnonzero((got != want).any(axis=1))
+    ctx.close()
+
+
 @pytest.mark.parametrize("head,C", [("f32", 4000), ("q8", 4000), ("f32", 4004)])
 def test_head_product_leaves_the_loss_turns_row_maxima(hip, orc, backend, head, C):
     """A relaxed head product right before the loss turn leaves its logits'
