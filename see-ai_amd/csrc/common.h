@@ -120,6 +120,43 @@ __device__ __forceinline__ float BlockSumF(float v, float* lds) {
   return r;
 }
 
+// The 64-row query blocks that reach a dK / dV workgroup's keys.  A query sees
+// keys from its document's start on, so with documents packed one after another
+// a block whose every start lies past the workgroup's last key adds nothing --
+// of 2048 tokens in documents of 400, three blocks in four.  `count` is -1 when
+// the blocks are to be walked as they are: the sequence's last row starts at 0
+// (no documents, as a rule: one load tells, and no scan is paid), or the list
+// does not hold them.  `start(row)` is the row's stored start, clamped.
+constexpr int kLiveMost = 512;
+struct LiveBlocks {
+  int count;
+  uint16_t idx[kLiveMost];
+};
+template <int kThreads, class Start>
+__device__ __forceinline__ int ListLiveBlocks(LiveBlocks& live, int S, int first, int n,
+                                              int last_key, Start&& start) {
+  if (Uniform(start(S - 1)) == 0 || n > kLiveMost) return -1;
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  for (int b = wave; b < n; b += kThreads / kWave) {
+    const int row = (first + b) * 64 + lane;
+    const bool any = __ballot(row < S && start(min(row, S - 1)) <= last_key) != 0;
+    if (lane == 0) live.idx[b] = any;
+  }
+  __syncthreads();
+  if (wave == 0) {  // the flags become the list, in place: it never runs ahead of them
+    int count = 0;
+    for (int b0 = 0; b0 < n; b0 += kWave) {
+      const bool any = b0 + lane < n && live.idx[b0 + lane] != 0;
+      const unsigned long long mask = __ballot(any);
+      if (any) live.idx[count + __popcll(mask & ((1ull << lane) - 1))] = static_cast<uint16_t>(b0 + lane);
+      count += __popcll(mask);
+    }
+    if (lane == 0) live.count = count;
+  }
+  __syncthreads();
+  return Uniform(live.count);
+}
+
 __device__ __forceinline__ float Bf16ToF32(uint16_t b) {
   return __uint_as_float(static_cast<uint32_t>(b) << 16);
 }

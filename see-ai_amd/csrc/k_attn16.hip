@@ -626,12 +626,18 @@ Attn16DKDV(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
     for (int s = 0; s < 4; ++s) kf[s] = OwnedFrag(krow, s, lane), vf[s] = OwnedFrag(vrow, s, lane);
   }
   const int blk_first = (kblk * kBwdRows) / kBlkRows;
-  const int nblk = (S + kBlkRows - 1) / kBlkRows - blk_first;
+  int nblk = (S + kBlkRows - 1) / kBlkRows - blk_first;
+  __shared__ LiveBlocks live;
+  const int nlive = ListLiveBlocks<kBwdWaves * kWave>(
+      live, S, blk_first, nblk, kblk * kBwdRows + kBwdRows - 1,
+      [&](int row) { return StatsStart(st_bh[row].w, row); });
+  if (nlive >= 0) nblk = nlive;
+  const auto block = [&](int ib) { return blk_first + (nlive >= 0 ? Uniform(live.idx[ib]) : ib); };
   int voff[4];
 #pragma unroll
   for (int jj = 0; jj < 4; ++jj) voff[jj] = TileLoadOffset((4 * jj + wave) % 8, lane, ld);
   auto issue = [&](int ib, uint8_t* sb) {
-    const int r0 = (blk_first + ib) * kBlkRows;
+    const int r0 = block(ib) * kBlkRows;
     const __amdgpu_buffer_rsrc_t rq = SliceRsrc(q + base, ld, S, r0);
     const __amdgpu_buffer_rsrc_t rd = SliceRsrc(dout + base, ld, S, r0);
 #pragma unroll
@@ -648,11 +654,11 @@ Attn16DKDV(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
   // a block's products.
   float4 pend = {};
   auto fetch = [&](int ib) {
-    const int iq = (blk_first + ib) * kBlkRows + lane;
+    const int iq = block(ib) * kBlkRows + lane;
     if (iq < S) pend = st_bh[iq];
   };
   auto put = [&](int ib, int buf) {
-    const int iq = (blk_first + ib) * kBlkRows + lane;
+    const int iq = block(ib) * kBlkRows + lane;
     int start = 0;
     if (iq < S) {
       Smm[buf][lane] = -RowOffset(pend.x, pend.y);
@@ -736,7 +742,7 @@ Attn16DKDV(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
       put(ib + 1, buf ^ 1);
       if (ib + 2 < nblk) fetch(ib + 2);
     }
-    const int r0 = (blk_first + ib) * kBlkRows;
+    const int r0 = block(ib) * kBlkRows;
     const int smax = Uniform(Smax[buf]);
 #pragma unroll
     for (int qt = 0; qt < 2; ++qt) {

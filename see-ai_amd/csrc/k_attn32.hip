@@ -467,7 +467,14 @@ Attn32DKDV(const float* __restrict__ q, const float* __restrict__ k, const float
 #pragma unroll
     for (int dt = 0; dt < D / 16; ++dt) dka[t][dt] = dva[t][dt] = v4f{0.f, 0.f, 0.f, 0.f};
 
-  const int qb0 = (rb * kRowsWG) / kBlk, qb1 = (S - 1) / kBlk;
+  const int qb0 = (rb * kRowsWG) / kBlk;
+  int nqb = (S - 1) / kBlk - qb0 + 1;
+  __shared__ LiveBlocks live;
+  const int nlive = ListLiveBlocks<kThreads>(
+      live, S, qb0, nqb, rb * kRowsWG + kRowsWG - 1,
+      [&](int row) { return StartOf(st_unit[static_cast<size_t>(row) * 4 + 3], row); });
+  if (nlive >= 0) nqb = nlive;
+  const auto block = [&](int n) { return qb0 + (nlive >= 0 ? Uniform(live.idx[n]) : n); };
   Block<D> nq, nd;
   float4 nst = make_float4(0.f, 0.f, 0.f, 0.f);
   auto load = [&](int qb) {
@@ -482,12 +489,12 @@ Attn32DKDV(const float* __restrict__ q, const float* __restrict__ k, const float
     nd.Store(lds[buf][1], tid);
     if (tid < kBlk) sst[buf][tid] = nst;
   };
-  load(qb0);
+  load(block(0));
   store(0);
   __syncthreads();
-  for (int qb = qb0; qb <= qb1; ++qb) {
-    const int buf = (qb - qb0) & 1;
-    if (qb < qb1) load(qb + 1);
+  for (int n = 0; n < nqb; ++n) {
+    const int buf = n & 1, qb = block(n);
+    if (n + 1 < nqb) load(block(n + 1));
     const float* Qs = lds[buf][0];
     const float* Ds = lds[buf][1];
     const int i0 = qb * kBlk;
@@ -526,7 +533,7 @@ Attn32DKDV(const float* __restrict__ q, const float* __restrict__ k, const float
           }
       }
     }
-    if (qb < qb1) store(buf ^ 1);
+    if (n + 1 < nqb) store(buf ^ 1);
     __syncthreads();
   }
 #pragma unroll

@@ -569,12 +569,18 @@ FlashDKDV(const float* __restrict__ q, const float* __restrict__ k, const float*
   if (kDK) LoadOwned<D>(v + base + static_cast<size_t>(jc) * ld, g, 1.0f, vf);
 
   const int blk_first = (kblk * kRows) / kBlk;
-  const int nblk = (S + kBlk - 1) / kBlk - blk_first;
+  int nblk = (S + kBlk - 1) / kBlk - blk_first;
+  __shared__ LiveBlocks live;
+  const int nlive = ListLiveBlocks<kFThreads>(
+      live, S, blk_first, nblk, kblk * kRows + kRows - 1,
+      [&](int row) { return static_cast<int>(StatsStart(st_bh[row].w, row)); });
+  if (nlive >= 0) nblk = nlive;
+  const auto block = [&](int ib) { return blk_first + (nlive >= 0 ? Uniform(live.idx[ib]) : ib); };
   const uint32_t ld32 = static_cast<uint32_t>(ld);
   const uint32_t slice_bytes = static_cast<uint32_t>(((S - 1) * ld + D) * 4);
   St sq(ld32), sd(ld32);
   auto load = [&](int ib) {
-    const int r0 = (blk_first + ib) * kBlk;
+    const int r0 = block(ib) * kBlk;
     sq.load(q + base, slice_bytes, ld32, r0);
     sd.load(dout + base, slice_bytes, ld32, r0);
   };
@@ -582,7 +588,7 @@ FlashDKDV(const float* __restrict__ q, const float* __restrict__ k, const float*
     sq.store(Qs[buf], kDK ? Qt[buf] : nullptr);
     sd.store(kDK ? Ds[buf] : nullptr, kDV ? Dt[buf] : nullptr);
     if (threadIdx.x < kBlk) {  // wave 0
-      const int t = threadIdx.x, iq = (blk_first + ib) * kBlk + t;
+      const int t = threadIdx.x, iq = block(ib) * kBlk + t;
       int start = 0;
       if (iq < S) {
         const float4 s4 = st_bh[iq];
@@ -646,7 +652,7 @@ FlashDKDV(const float* __restrict__ q, const float* __restrict__ k, const float*
   for (int ib = 0; ib < nblk; ++ib) {
     const int buf = ib & 1;
     if (ib + 1 < nblk) load(ib + 1);
-    const int r0 = (blk_first + ib) * kBlk;
+    const int r0 = block(ib) * kBlk;
     if (r0 >= j0w + 31 && r0 + kBlk <= S && Uniform(Smax[buf]) <= j0w)
       run(std::false_type{}, buf, r0);
     else if (r0 + kBlk - 1 >= j0w)  // some query of the block reaches this wave's keys

@@ -558,6 +558,82 @@ def test_head_product_leaves_the_loss_turns_row_maxima(hip, orc, backend, head, 
         assert e <= TOL_BF16, f"{name}: {e:.3g}"
 
 
+def _document_starts(kind, B, S):
+    """First keys per token: packed documents of mixed lengths; starts in no
+    order; packed documents whose last row starts at 0 (its blocks are walked
+    without the list)."""
+    r = rng(B * S)
+    out = np.zeros((B, S), np.int32)
+    if kind == "unordered":
+        out[:] = r.integers(0, np.arange(S) + 1)
+        out[:, -1] = S // 2
+        return out.reshape(-1)
+    for b in range(B):
+        at = 0
+        while at < S:
+            n = int(r.integers(1, 200))
+            out[b, at:at + n] = at
+            at += n
+    if kind == "last_open":
+        out[:, -1] = 0
+    return out.reshape(-1)
+
+
+@pytest.mark.parametrize("kind", ["packed", "unordered", "last_open"])
+@pytest.mark.parametrize("family,d", [("f32", 64), ("f32", 128), ("relaxed", 64), ("relaxed", 128),
+                                      ("bf16", 64)])
+def test_attention_backward_walks_the_documents_blocks(hip, torch_cuda, family, d, kind):
+    """dK and dV over packed documents, where most query blocks reach none of
+    a workgroup's keys, against float64 attention: 1e-5 (f32) and 2e-2 (bf16
+    products), per tensor."""
+    torch = torch_cuda
+    B, S, H = 2, 709, 3
+    print(f"attention documents {family} d={d} {kind}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(d)
+    q, k, v, do = (torch.randn((B * S, H * d), device="cuda", generator=g) for _ in range(4))
+    if family == "bf16":
+        q, k, v, do = (t.to(torch.bfloat16) for t in (q, k, v, do))
+    starts = torch.from_numpy(_document_starts(kind, B, S)).cuda()
+    new = lambda: torch.full((B * S, H * d), float("nan"), device="cuda")  # noqa: E731
+    o, dq, dk, dv = new(), new(), new(), new()
+    st = torch.empty((B * H * S, 4), device="cuda")
+    P = lambda t: t.data_ptr()  # noqa: E731
+    ctx = hip.Context(0)
+    ctx.use_torch_stream()
+    geo = (B, S, H, d)
+    if family == "bf16":
+        ctx.call("seeai_attn_fwd_bf16", P(q), P(k), P(v), P(o), P(st), *geo, P(starts))
+        ctx.call("seeai_attn_dq_bf16", P(q), P(k), P(v), P(do), P(st), P(dq), *geo)
+        ctx.call("seeai_attn_dkdv_bf16", P(q), P(k), P(v), P(do), P(st), P(dk), P(dv), *geo)
+    else:
+        dt = int(family == "relaxed")
+        ctx.call("seeai_attn_fwd", dt, P(q), P(k), P(v), P(o), P(st), *geo, P(starts))
+        ctx.call("seeai_attn_dq", dt, P(q), P(k), P(v), P(do), P(st), P(dq), *geo)
+        if dt == 0:
+            ctx.call("seeai_attn_dkdv_f32", P(q), P(k), P(v), P(do), P(st), P(dk), P(dv), *geo)
+        elif d == 64:
+            ctx.call("seeai_attn_dkdv", P(q), P(k), P(v), P(do), P(st), P(dk), P(dv), *geo)
+        else:
+            ctx.call("seeai_attn_dk", dt, P(q), P(k), P(v), P(do), P(st), P(dk), *geo)
+            ctx.call("seeai_attn_dv", dt, P(q), P(k), P(do), P(st), P(dv), *geo)
+    torch.cuda.synchronize()
+    ctx.close()
+    split = lambda t: t.double().view(B, S, H, d).transpose(1, 2).contiguous()  # noqa: E731
+    i = torch.arange(S, device="cuda")
+    ok = (i[None, :] <= i[:, None])[None, None] & (i >= starts.view(B, 1, S, 1))
+    Q, K, V, G = split(q), split(k), split(v), split(do)
+    sc = (Q @ K.transpose(2, 3).contiguous() / d ** 0.5).masked_fill(~ok, -float("inf"))
+    p = torch.softmax(sc, dim=3)
+    dp = G @ V.transpose(2, 3).contiguous()
+    ds = p * (dp - (p * dp).sum(dim=3, keepdim=True)) / d ** 0.5
+    want = {"o": p @ V, "dq": ds @ K, "dk": ds.transpose(2, 3).contiguous() @ Q,
+            "dv": p.transpose(2, 3).contiguous() @ G}
+    bar = TOL if family == "f32" else TOL_BF16
+    for name, got in [("o", o), ("dq", dq), ("dk", dk), ("dv", dv)]:
+        e = float((split(got) - want[name]).abs().max() / want[name].abs().max())
+        assert e <= bar, f"{name}: {e:.3g}"
+
+
 # --- optimizer -----------------------------------------------------------------------------
 
 @pytest.mark.parametrize("n", [1, 2048, 100003])
