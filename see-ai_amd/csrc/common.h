@@ -477,6 +477,13 @@ hipError_t LaunchAttnDVTiled(int dtype, const float* q, const float* k, const fl
 // through LDS (k_attn32.hip).  In LaunchAttn32DKDV one or both of dk, dv are
 // non-null; each output has the same bits either way.
 bool Attn32Fits(size_t B, size_t S, size_t H, size_t d, std::initializer_list<const void*> ptrs);
+hipError_t LaunchAttn3Fwd(const float* q, const float* k, const float* v, float* o, float* stats,
+                          size_t B, size_t S, size_t H, const int32_t* starts, hipStream_t s);
+hipError_t LaunchAttn3DQ(const float* q, const float* k, const float* v, const float* dout,
+                         float* stats, float* dq, size_t B, size_t S, size_t H, hipStream_t s);
+hipError_t LaunchAttn3DKDV(const float* q, const float* k, const float* v, const float* dout,
+                           const float* stats, float* dk, float* dv, size_t B, size_t S, size_t H,
+                           hipStream_t s);
 hipError_t LaunchAttn32Fwd(const float* q, const float* k, const float* v, float* o, float* stats,
                            size_t B, size_t S, size_t H, size_t d, const int32_t* starts,
                            hipStream_t s);

@@ -1,0 +1,500 @@
+// k_attn3.hip -- the exact family of causal attention (kAttnFwdTiled,
+// kAttnDQTiled, kAttnDKTiled, kAttnDVTiled; source/plan/instruction.h:
+// 158-259) at head width 64: f32 products formed on bf16 MFMA.  The
+// reference's expressions per score (attention.cc:405-590): s = (q . k) /
+// sqrt(d), p = exp(s - m) * (1/l), delta = sum_j p dP (in double), dS =
+// p (dP - delta), dQ += (dS / sqrt(d)) k, dK += (dS / sqrt(d)) q, dV += p dO.
+//
+// Products.  Every f32 operand is split three ways, x = h + m + l, each part
+// the bf16 nearest to what is left: 8 + 8 + 8 significant bits, so the parts
+// hold x (to the last bit or so).  A product sums six of the nine part
+// products -- hh in the accumulator, hm, mh, mm, hl, lh in one of their own
+// that joins it at the end; the three left out are below 2^-26 of the operands'
+// product -- each exact in the MFMA, summed in f32.  Against float64 the
+// results are as close as sums of v_mfma_f32_16x16x4f32 (a chain of rounded
+// f32 terms) or closer: fewer roundings at the accumulator's magnitude.  Six
+// bf16 products take 3/8 of the f32 MFMA's time, which bounded these kernels
+// (v_mfma_f32_16x16x4f32 at 55-60 % of its rate).  us, f32 MFMA / here:
+//
+//   B8 H12 S1024     forward 184 / 108   dQ 408 / 224    dK + dV 342 / 270
+//   B16 H16 S2048            1491 / 878     3627 / 1805          3258 / 2245
+//   B1 H8 S328                 43 / 26        94 / 40              65 / 51
+//
+// 2-norm error against float64 at B2 H4 S1024, unit normals, f32 MFMA / here:
+// O 3.2e-7 / 1.4e-7, dQ 3.9e-7 / 1.8e-7, dK 7.6e-7 / 3.1e-7, dV 7.4e-7 /
+// 3.1e-7; with scores of standard deviation 8, dQ 1.9e-6 / 9.9e-7.  What bounds
+// them now is a wave's own chain (products, exps, splits) at two waves a SIMD
+// (one for dQ and dK / dV): MFMA busy 23 %, VALU 32 % of the forward.
+//
+// Geometry.  A workgroup of four waves owns 128 rows of one (b, h) -- queries
+// for the forward and dQ, keys for dK / dV -- each wave 32 of them, their parts
+// held as MFMA fragments.  The other side streams in 64-row blocks, split once
+// as it is staged into three bf16 tiles in LDS; one buffer (48 KiB for the
+// pair) and the next block in flight in registers, so two of the forward's
+// workgroups share a CU and one multiplies while the other stages.  Tiles, fragments and the
+// transposed score layout are k_attn16.hip's.
+//
+// Every output element has one writer and every sum a fixed order; dK and dV
+// are one template, so the fused pass has the separate passes' bits.
+#include "attn_tile.h"
+
+namespace seeai {
+namespace {
+
+constexpr int kWaves = 4, kThreads = kWaves * kWave, kRowsWG = kWaves * 32;
+constexpr float kIsd = 0.125f;  // 1 / sqrt(64)
+
+// instruction.h:240-247: a stored start clamped into [0, i], NaN to 0.
+__device__ __forceinline__ int StartOf(float stored, int i) {
+  if (!(stored > 0.0f)) return 0;
+  const float cap = static_cast<float>(i);
+  return stored >= cap ? i : static_cast<int>(stored);
+}
+
+// Workgroup w -> (b, h) and its row block's rank, the longest first over all
+// (b, h); with B H a multiple of 8 every block of a slice lands on one XCD (the
+// hardware deals workgroups to XCDs round-robin).
+__device__ __forceinline__ void UnitOf3(int nb, int& bh, int& rank) {
+  const int units = gridDim.x / nb;
+  bh = blockIdx.x % units;
+  rank = blockIdx.x / units;
+}
+
+struct Parts {
+  bf16x8 p[3];  // h, m, l
+};
+// Eight floats in their parts.  kFinite: no infinities among them; otherwise
+// an infinity is its own first part and the rest is zero.
+template <bool kFinite>
+__device__ __forceinline__ Parts Split(const float (&x)[8]) {
+  Parts r;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    r.p[0][i] = static_cast<__bf16>(x[i]);
+    float rest = x[i] - static_cast<float>(r.p[0][i]);
+    if (!kFinite) rest = rest == rest ? rest : 0.0f;
+    r.p[1][i] = static_cast<__bf16>(rest);
+    r.p[2][i] = static_cast<__bf16>(rest - static_cast<float>(r.p[1][i]));
+  }
+  return r;
+}
+
+// hi += hh, lo += the five smaller part products.
+__device__ __forceinline__ void Mfma3(const Parts& a, const Parts& b, v16f& hi, v16f& lo) {
+  lo = Mfma(a.p[0], b.p[2], lo);
+  lo = Mfma(a.p[2], b.p[0], lo);
+  lo = Mfma(a.p[1], b.p[1], lo);
+  lo = Mfma(a.p[0], b.p[1], lo);
+  lo = Mfma(a.p[1], b.p[0], lo);
+  hi = Mfma(a.p[0], b.p[0], hi);
+}
+
+// One staged 64-row block: its floats in flight, then its three tiles.
+struct Tile3 {
+  uint8_t part[3][kTile];
+};
+struct Block3 {
+  float4 r[4];  // two chunks of eight dims: rows tid / 8 and 32 + tid / 8, chunk tid % 8
+
+  __device__ __forceinline__ void Load(const float* __restrict__ base, size_t ld, int row0, int S) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int row = row0 + e * 32 + static_cast<int>(threadIdx.x) / 8;
+      const float* p = base + static_cast<size_t>(min(row, S - 1)) * ld + threadIdx.x % 8 * 8;
+      r[2 * e] = *reinterpret_cast<const float4*>(p);
+      r[2 * e + 1] = *reinterpret_cast<const float4*>(p + 4);
+    }
+  }
+  // Rows past the sequence are left as its last row: their scores are masked.
+  __device__ __forceinline__ void Store(Tile3& t) const {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int row = e * 32 + threadIdx.x / 8, ch = threadIdx.x % 8;
+      const float x[8] = {r[2 * e].x,     r[2 * e].y,     r[2 * e].z,     r[2 * e].w,
+                          r[2 * e + 1].x, r[2 * e + 1].y, r[2 * e + 1].z, r[2 * e + 1].w};
+      const Parts s = Split<false>(x);
+      const int at = ch / 4 * kHalf + row * 64 + Phys(row, ch % 4) * 16;
+#pragma unroll
+      for (int p = 0; p < 3; ++p) *reinterpret_cast<bf16x8*>(t.part[p] + at) = s.p[p];
+    }
+  }
+};
+
+// This lane's fragments of one own row: dims 16 s + 8 g .. + 8, s < 4.
+__device__ __forceinline__ void OwnParts(const float* __restrict__ row, int lane, Parts (&f)[4]) {
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const float* p = row + 16 * s + 8 * (lane / 32);
+    const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
+    const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    f[s] = Split<false>(x);
+  }
+}
+__device__ __forceinline__ Parts RowParts(const Tile3& t, const FragOffsets& fo, int row0, int s) {
+  return Parts{{RowFrag(t.part[0], fo, row0, s), RowFrag(t.part[1], fo, row0, s),
+                RowFrag(t.part[2], fo, row0, s)}};
+}
+__device__ __forceinline__ Parts ColParts(const Tile3& t, const FragOffsets& fo, int dt, int k0) {
+  return Parts{{ColFrag(t.part[0], fo, dt, k0), ColFrag(t.part[1], fo, dt, k0),
+                ColFrag(t.part[2], fo, dt, k0)}};
+}
+// Staged rows row0 .. + 32 against the own rows, over the 64 dims: lane (g, c)
+// gets rows 8q + 4g + e against own row c.
+__device__ __forceinline__ v16f Dot3(const Tile3& t, const FragOffsets& fo, int row0,
+                                     const Parts (&own)[4]) {
+  v16f hi = {}, lo = {};
+#pragma unroll
+  for (int s = 0; s < 4; ++s) Mfma3(RowParts(t, fo, row0, s), own[s], hi, lo);
+  return hi + lo;
+}
+// acc[dt] += (the tile's columns 32 dt ..)^T over rows row0 .. + 32 times w,
+// the rows' values in score order.
+__device__ __forceinline__ void Accum3(const Tile3& t, const FragOffsets& fo, int row0,
+                                       const float (&w)[16], v16f (&acc)[2]) {
+  Parts b[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const float x[8] = {w[8 * h],     w[8 * h + 1], w[8 * h + 2], w[8 * h + 3],
+                        w[8 * h + 4], w[8 * h + 5], w[8 * h + 6], w[8 * h + 7]};
+    b[h] = Split<true>(x);
+  }
+#pragma unroll
+  for (int dt = 0; dt < 2; ++dt) {
+    v16f lo = {};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) Mfma3(ColParts(t, fo, dt, row0 + 16 * h), b[h], acc[dt], lo);
+    acc[dt] += lo;
+  }
+}
+
+// exp(y) by the hardware's exp2: y is a rounded difference from the row's
+// maximum, so y log2(e) errs by 2^-24 of itself, as far as y's own rounding.
+__device__ __forceinline__ float ExpOf(float y) { return Exp2(y * kLog2e); }
+
+__device__ __forceinline__ void StoreRow(float* row, int g, const v16f (&acc)[2], float scale) {
+#pragma unroll
+  for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      *reinterpret_cast<float4*>(row + 32 * dt + 8 * q + 4 * g) =
+          make_float4(acc[dt][4 * q] * scale, acc[dt][4 * q + 1] * scale,
+                      acc[dt][4 * q + 2] * scale, acc[dt][4 * q + 3] * scale);
+}
+
+// The key range of a workgroup's queries: from the earliest start to the last
+// query, in blocks.
+__device__ __forceinline__ void KeyBlocks(int start, int i0, int S, int& first, int& count) {
+  __shared__ int lo[kWaves];
+  const int l = WaveMinI(start);
+  if (threadIdx.x % kWave == 0) lo[threadIdx.x / kWave] = l;
+  __syncthreads();
+  first = min(min(lo[0], lo[1]), min(lo[2], lo[3])) / kBlkRows;
+  count = min(i0 + kRowsWG - 1, S - 1) / kBlkRows - first + 1;
+}
+
+// ---------------------------------------------------------------------------
+// Forward (attention.cc:448-493): online softmax over 64-key blocks; the stats
+// row gets the row max, 1/l, 0 and the clamped start.
+// ---------------------------------------------------------------------------
+__global__ void __launch_bounds__(kThreads, 2)
+Attn3Fwd(const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
+         float* __restrict__ o, float* __restrict__ stats, int S, int H,
+         const int32_t* __restrict__ starts) {
+  __shared__ __attribute__((aligned(1024))) Tile3 kt, vt;
+  const int lane = threadIdx.x % kWave, g = lane / 32;
+  const int wave = Uniform(threadIdx.x / kWave);
+  const int nb = (S + kRowsWG - 1) / kRowsWG;
+  int bh, rank;
+  UnitOf3(nb, bh, rank);
+  const int b = bh / H, h = bh % H;
+  const size_t ld = static_cast<size_t>(H) * kD;
+  const size_t base = static_cast<size_t>(b) * S * ld + static_cast<size_t>(h) * kD;
+  const int i0 = (nb - 1 - rank) * kRowsWG, iw = i0 + wave * 32, i = iw + lane % 32;
+  const int ic = min(i, S - 1);
+  int start = 0;
+  if (starts) {
+    const int s0 = starts[static_cast<size_t>(b) * S + ic];
+    start = s0 <= 0 ? 0 : (s0 < ic ? s0 : ic);
+  }
+  int jb0, nblk;
+  KeyBlocks(start, i0, S, jb0, nblk);
+  const int wave_last = min(iw + 31, S - 1), wave_start = WaveMaxI(start);
+  Parts qf[4];
+  OwnParts(q + base + static_cast<size_t>(ic) * ld, lane, qf);
+
+  const FragOffsets fo = MakeFragOffsets(lane);
+  v16f acc[2] = {};
+  float m = -INFINITY, l = 0.0f;  // l: this half's share
+  Block3 nk, nv;
+  nk.Load(k + base, ld, jb0 * kBlkRows, S);
+  nv.Load(v + base, ld, jb0 * kBlkRows, S);
+  for (int n = 0; n < nblk; ++n) {
+    const int j0 = (jb0 + n) * kBlkRows;
+    if (n > 0) __syncthreads();  // the last block's reads are done
+    nk.Store(kt);
+    nv.Store(vt);
+    __syncthreads();
+    if (n + 1 < nblk) {
+      nk.Load(k + base, ld, j0 + kBlkRows, S);
+      nv.Load(v + base, ld, j0 + kBlkRows, S);
+    }
+    if (j0 > wave_last) continue;
+    float p[2][16];
+    float mx = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int jt = j0 + 32 * t;
+      if (jt > wave_last) {  // wave-uniform: wholly above the diagonal
+#pragma unroll
+        for (int r = 0; r < 16; ++r) p[t][r] = -INFINITY;
+        continue;
+      }
+      const v16f sc = Dot3(kt, fo, 32 * t, qf);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) p[t][r] = sc[r] * kIsd;
+      if (!(jt + 31 <= iw && jt >= wave_start && iw + 31 < S)) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int j = jt + RowConst(r) + 4 * g;
+          p[t][r] = j <= i && j >= start && i < S ? p[t][r] : -INFINITY;
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, p[t][r]);
+    }
+    const float mn = fmaxf(m, SwapMax(mx));
+    const float ref = mn == -INFINITY ? 0.0f : mn;
+    const float alpha = m == -INFINITY ? 0.0f : ExpOf(m - ref);
+    float sum = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        p[t][r] = ExpOf(p[t][r] - ref);
+        sum += p[t][r];
+      }
+    l = l * alpha + sum;
+    m = mn;
+    acc[0] *= alpha;
+    acc[1] *= alpha;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+      if (j0 + 32 * t <= wave_last) Accum3(vt, fo, 32 * t, p[t], acc);
+  }
+  if (i >= S) return;
+  const float inv = 1.0f / SwapSum(l);
+  StoreRow(o + base + static_cast<size_t>(i) * ld, g, acc, inv);
+  if (g == 0)
+    *reinterpret_cast<float4*>(stats + (static_cast<size_t>(bh) * S + i) * 4) =
+        make_float4(m, inv, 0.0f, static_cast<float>(start));
+}
+
+// ---------------------------------------------------------------------------
+// dQ (attention.cc:495-535) in one walk over the keys: dS = p (dP - delta) is
+// linear in delta, so dQ = (sum p dP k - delta sum p k) / sqrt(d) with delta =
+// sum p dP (in double) from the same walk -- four products and one exponential
+// a score where a walk for delta and one for dQ take five and two (395 us at
+// B8 H12 S1024, two walks, 224 us here), and its error against float64 stays
+// below half the f32 MFMA kernel's two-walk form's.
+// ---------------------------------------------------------------------------
+__global__ void __launch_bounds__(kThreads, 1)
+Attn3DQ(const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
+        const float* __restrict__ dout, float* __restrict__ stats, float* __restrict__ dq, int S,
+        int H) {
+  __shared__ __attribute__((aligned(1024))) Tile3 kt, vt;
+  const int lane = threadIdx.x % kWave, g = lane / 32;
+  const int wave = Uniform(threadIdx.x / kWave);
+  const int nb = (S + kRowsWG - 1) / kRowsWG;
+  int bh, rank;
+  UnitOf3(nb, bh, rank);
+  const int b = bh / H, h = bh % H;
+  const size_t ld = static_cast<size_t>(H) * kD;
+  const size_t base = static_cast<size_t>(b) * S * ld + static_cast<size_t>(h) * kD;
+  const int i0 = (nb - 1 - rank) * kRowsWG, iw = i0 + wave * 32, i = iw + lane % 32;
+  const int ic = min(i, S - 1);
+  const float4 st = *reinterpret_cast<const float4*>(stats + (static_cast<size_t>(bh) * S + ic) * 4);
+  const int start = StartOf(st.w, ic);
+  int jb0, nblk;
+  KeyBlocks(start, i0, S, jb0, nblk);
+  const int wave_last = min(iw + 31, S - 1), wave_start = WaveMaxI(start);
+  Parts qf[4], df[4];
+  OwnParts(q + base + static_cast<size_t>(ic) * ld, lane, qf);
+  OwnParts(dout + base + static_cast<size_t>(ic) * ld, lane, df);
+
+  const FragOffsets fo = MakeFragOffsets(lane);
+  v16f acc_d[2] = {}, acc_p[2] = {};  // sums of (p dP) k and of p k
+  double dsum = 0.0;
+  Block3 nk, nv;
+  nk.Load(k + base, ld, jb0 * kBlkRows, S);
+  nv.Load(v + base, ld, jb0 * kBlkRows, S);
+  for (int n = 0; n < nblk; ++n) {
+    const int j0 = (jb0 + n) * kBlkRows;
+    if (n > 0) __syncthreads();
+    nk.Store(kt);
+    nv.Store(vt);
+    __syncthreads();
+    if (n + 1 < nblk) {
+      nk.Load(k + base, ld, j0 + kBlkRows, S);
+      nv.Load(v + base, ld, j0 + kBlkRows, S);
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int jt = j0 + 32 * t;
+      if (jt > wave_last) continue;  // wave-uniform
+      const v16f sc = Dot3(kt, fo, 32 * t, qf), dp = Dot3(vt, fo, 32 * t, df);
+      float p[16], w[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) p[r] = ExpOf(sc[r] * kIsd - st.x) * st.y;
+      if (!(jt + 31 <= iw && jt >= wave_start && iw + 31 < S)) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int j = jt + RowConst(r) + 4 * g;
+          p[r] = j <= i && j >= start && i < S ? p[r] : 0.0f;
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        w[r] = p[r] != 0.0f ? p[r] * dp[r] : 0.0f;
+        if (p[r] != 0.0f) dsum += static_cast<double>(dp[r]) * p[r];
+      }
+      Accum3(kt, fo, 32 * t, w, acc_d);
+      Accum3(kt, fo, 32 * t, p, acc_p);
+    }
+  }
+  const float delta = static_cast<float>(dsum + __shfl_xor(dsum, 32, kWave));
+  v16f acc[2];
+#pragma unroll
+  for (int dt = 0; dt < 2; ++dt) acc[dt] = (acc_d[dt] - delta * acc_p[dt]) * kIsd;
+  if (i >= S) return;
+  StoreRow(dq + base + static_cast<size_t>(i) * ld, g, acc, 1.0f);
+  if (g == 0) stats[(static_cast<size_t>(bh) * S + i) * 4 + 2] = delta;
+}
+
+// ---------------------------------------------------------------------------
+// dK and dV (attention.cc:537-590): each wave's 32 keys against 64-query
+// blocks from the diagonal down.  kDK / kDV pick the outputs; each output's
+// arithmetic is the same whichever else is formed.
+// ---------------------------------------------------------------------------
+template <bool kDK, bool kDV>
+__global__ void __launch_bounds__(kThreads, kDK ? 1 : 2)
+Attn3DKDV(const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
+          const float* __restrict__ dout, const float* __restrict__ stats, float* __restrict__ dk,
+          float* __restrict__ dv, int S, int H) {
+  __shared__ __attribute__((aligned(1024))) Tile3 qt, dt;
+  // Per staged query: m, 1/l, delta, and its first key.
+  __shared__ __attribute__((aligned(16))) float sm[kBlkRows], si[kBlkRows], sd[kBlkRows];
+  __shared__ __attribute__((aligned(16))) int ss[kBlkRows];
+  __shared__ int smax;
+  __shared__ LiveBlocks live;
+  const int lane = threadIdx.x % kWave, g = lane / 32;
+  const int wave = Uniform(threadIdx.x / kWave);
+  const int nb = (S + kRowsWG - 1) / kRowsWG;
+  int bh, rank;
+  UnitOf3(nb, bh, rank);  // rank 0: the first keys, the longest columns
+  const int b = bh / H, h = bh % H;
+  const size_t ld = static_cast<size_t>(H) * kD;
+  const size_t base = static_cast<size_t>(b) * S * ld + static_cast<size_t>(h) * kD;
+  const int jw = rank * kRowsWG + wave * 32, j = jw + lane % 32, jc = min(j, S - 1);
+  const float4* st = reinterpret_cast<const float4*>(stats) + static_cast<size_t>(bh) * S;
+  const int qb0 = rank * kRowsWG / kBlkRows;
+  int nblk = (S - 1) / kBlkRows - qb0 + 1;
+  const int nlive = ListLiveBlocks<kThreads>(live, S, qb0, nblk, rank * kRowsWG + kRowsWG - 1,
+                                             [&](int row) { return StartOf(st[row].w, row); });
+  if (nlive >= 0) nblk = nlive;
+  const auto block = [&](int n) { return qb0 + (nlive >= 0 ? Uniform(live.idx[n]) : n); };
+
+  Parts kf[4], vf[kDK ? 4 : 1];
+  OwnParts(k + base + static_cast<size_t>(jc) * ld, lane, kf);
+  if constexpr (kDK) OwnParts(v + base + static_cast<size_t>(jc) * ld, lane, vf);
+  const FragOffsets fo = MakeFragOffsets(lane);
+  v16f acc_k[2] = {}, acc_v[2] = {};
+  Block3 nq, nd;
+  float4 ns = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto load = [&](int qb) {
+    nq.Load(q + base, ld, qb * kBlkRows, S);
+    nd.Load(dout + base, ld, qb * kBlkRows, S);
+    if (threadIdx.x < kBlkRows) ns = st[min(qb * kBlkRows + static_cast<int>(threadIdx.x), S - 1)];
+  };
+  const auto rows = [&](const auto* terms, int t, int r) { return terms[32 * t + RowConst(r) + 4 * g]; };
+  load(block(0));
+  for (int n = 0; n < nblk; ++n) {
+    const int i0 = block(n) * kBlkRows;
+    if (n > 0) __syncthreads();
+    nq.Store(qt);
+    nd.Store(dt);
+    if (wave == 0) {
+      const int start = StartOf(ns.w, min(i0 + lane, S - 1));
+      sm[lane] = ns.x, si[lane] = ns.y, sd[lane] = ns.z, ss[lane] = start;
+      const int mx = WaveMaxI(start);
+      if (lane == 0) smax = mx;
+    }
+    __syncthreads();
+    if (n + 1 < nblk) load(block(n + 1));
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int it = i0 + 32 * t;
+      if (it >= S || it + 31 < jw) continue;  // wave-uniform: no query sees a key
+      const v16f sc = Dot3(qt, fo, 32 * t, kf);
+      float p[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        p[r] = ExpOf(sc[r] * kIsd - rows(sm, t, r)) * rows(si, t, r);
+      if (!(it >= jw + 31 && it + 31 < S && Uniform(smax) <= jw)) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int i = it + RowConst(r) + 4 * g;
+          p[r] = i < S && j <= i && j >= rows(ss, t, r) ? p[r] : 0.0f;
+        }
+      }
+      if constexpr (kDV) Accum3(dt, fo, 32 * t, p, acc_v);
+      if constexpr (kDK) {
+        const v16f dp = Dot3(dt, fo, 32 * t, vf);
+        float w[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          w[r] = p[r] != 0.0f ? (p[r] * (dp[r] - rows(sd, t, r))) * kIsd : 0.0f;
+        Accum3(qt, fo, 32 * t, w, acc_k);
+      }
+    }
+  }
+  if (j >= S) return;
+  const size_t at = base + static_cast<size_t>(j) * ld;
+  if constexpr (kDK) StoreRow(dk + at, g, acc_k, 1.0f);
+  if constexpr (kDV) StoreRow(dv + at, g, acc_v, 1.0f);
+}
+
+dim3 GridOf(size_t B, size_t S, size_t H) {
+  return dim3(static_cast<unsigned>((S + kRowsWG - 1) / kRowsWG * B * H));
+}
+
+}  // namespace
+
+hipError_t LaunchAttn3Fwd(const float* q, const float* k, const float* v, float* o, float* stats,
+                          size_t B, size_t S, size_t H, const int32_t* starts, hipStream_t s) {
+  hipLaunchKernelGGL(Attn3Fwd, GridOf(B, S, H), dim3(kThreads), 0, s, q, k, v, o, stats,
+                     static_cast<int>(S), static_cast<int>(H), starts);
+  return hipGetLastError();
+}
+
+hipError_t LaunchAttn3DQ(const float* q, const float* k, const float* v, const float* dout,
+                         float* stats, float* dq, size_t B, size_t S, size_t H, hipStream_t s) {
+  hipLaunchKernelGGL(Attn3DQ, GridOf(B, S, H), dim3(kThreads), 0, s, q, k, v, dout, stats, dq,
+                     static_cast<int>(S), static_cast<int>(H));
+  return hipGetLastError();
+}
+
+hipError_t LaunchAttn3DKDV(const float* q, const float* k, const float* v, const float* dout,
+                           const float* stats, float* dk, float* dv, size_t B, size_t S, size_t H,
+                           hipStream_t s) {
+  const int Si = static_cast<int>(S), Hi = static_cast<int>(H);
+#define SEEAI_DKDV(K, V)                                                                         \
+  hipLaunchKernelGGL((Attn3DKDV<K, V>), GridOf(B, S, H), dim3(kThreads), 0, s, q, k, v, dout, stats, \
+                     dk, dv, Si, Hi)
+  if (dk && dv) SEEAI_DKDV(true, true);
+  else if (dk) SEEAI_DKDV(true, false);
+  else SEEAI_DKDV(false, true);
+#undef SEEAI_DKDV
+  return hipGetLastError();
+}
+
+}  // namespace seeai

@@ -1,7 +1,7 @@
 // k_attn32.hip -- the exact family of causal attention (kAttnFwdTiled,
 // kAttnDQTiled, kAttnDKTiled, kAttnDVTiled; source/plan/instruction.h:
-// 158-259) on f32 operands, on v_mfma_f32_16x16x4f32, head widths 64 and
-// 128.  The reference's expressions per score (attention.cc:405-590, the
+// 158-259) on f32 operands, on v_mfma_f32_16x16x4f32, at head width 128 (64
+// runs k_attn3.hip).  The reference's expressions per score (attention.cc:405-590, the
 // oracle's prob_of and unit loops): s = f32(q . k) * (1/sqrt(d)),
 // p = exp(s - m) * (1/l), delta = sum_j p dP (accumulated in double),
 // dS = p (dP - delta), dQ += (dS / sqrt(d)) k, dK += (dS / sqrt(d)) q,
@@ -569,45 +569,32 @@ bool Attn32Fits(size_t B, size_t S, size_t H, size_t d, std::initializer_list<co
 hipError_t LaunchAttn32Fwd(const float* q, const float* k, const float* v, float* o, float* stats,
                            size_t B, size_t S, size_t H, size_t d, const int32_t* starts,
                            hipStream_t s) {
-  const int Si = static_cast<int>(S), Hi = static_cast<int>(H);
-  if (d == 64)
-    hipLaunchKernelGGL(Attn32Fwd<64>, GridOf(B, S, H), dim3(kThreads), 0, s, q, k, v, o, stats, Si,
-                       Hi, starts);
-  else
-    hipLaunchKernelGGL(Attn32Fwd<128>, GridOf(B, S, H), dim3(kThreads), 0, s, q, k, v, o, stats,
-                       Si, Hi, starts);
+  if (d == 64) return LaunchAttn3Fwd(q, k, v, o, stats, B, S, H, starts, s);
+  hipLaunchKernelGGL(Attn32Fwd<128>, GridOf(B, S, H), dim3(kThreads), 0, s, q, k, v, o, stats,
+                     static_cast<int>(S), static_cast<int>(H), starts);
   return hipGetLastError();
 }
 
 hipError_t LaunchAttn32DQ(const float* q, const float* k, const float* v, const float* dout,
                           float* stats, float* dq, size_t B, size_t S, size_t H, size_t d,
                           hipStream_t s) {
-  const int Si = static_cast<int>(S), Hi = static_cast<int>(H);
-  if (d == 64)
-    hipLaunchKernelGGL(Attn32DQ<64>, GridOf(B, S, H), dim3(kThreads), 0, s, q, k, v, dout, stats,
-                       dq, Si, Hi);
-  else
-    hipLaunchKernelGGL(Attn32DQ<128>, GridOf(B, S, H), dim3(kThreads), 0, s, q, k, v, dout, stats,
-                       dq, Si, Hi);
+  if (d == 64) return LaunchAttn3DQ(q, k, v, dout, stats, dq, B, S, H, s);
+  hipLaunchKernelGGL(Attn32DQ<128>, GridOf(B, S, H), dim3(kThreads), 0, s, q, k, v, dout, stats,
+                     dq, static_cast<int>(S), static_cast<int>(H));
   return hipGetLastError();
 }
 
 hipError_t LaunchAttn32DKDV(const float* q, const float* k, const float* v, const float* dout,
                             const float* stats, float* dk, float* dv, size_t B, size_t S, size_t H,
                             size_t d, hipStream_t s) {
+  if (d == 64) return LaunchAttn3DKDV(q, k, v, dout, stats, dk, dv, B, S, H, s);
   const int Si = static_cast<int>(S), Hi = static_cast<int>(H);
   const dim3 grid = GridOf(B, S, H), blk(kThreads);
 #define SEEAI_DKDV(DD, A, Bv) \
   hipLaunchKernelGGL((Attn32DKDV<DD, A, Bv>), grid, blk, 0, s, q, k, v, dout, stats, dk, dv, Si, Hi)
-  if (d == 64) {
-    if (dk && dv) SEEAI_DKDV(64, true, true);
-    else if (dk) SEEAI_DKDV(64, true, false);
-    else SEEAI_DKDV(64, false, true);
-  } else {
-    if (dk && dv) SEEAI_DKDV(128, true, true);
-    else if (dk) SEEAI_DKDV(128, true, false);
-    else SEEAI_DKDV(128, false, true);
-  }
+  if (dk && dv) SEEAI_DKDV(128, true, true);
+  else if (dk) SEEAI_DKDV(128, true, false);
+  else SEEAI_DKDV(128, false, true);
 #undef SEEAI_DKDV
   return hipGetLastError();
 }

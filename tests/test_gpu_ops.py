@@ -634,6 +634,51 @@ def test_attention_backward_walks_the_documents_blocks(hip, torch_cuda, family, 
         assert e <= bar, f"{name}: {e:.3g}"
 
 
+@pytest.mark.parametrize("S", [1, 31, 64, 65, 129, 300])
+@pytest.mark.parametrize("spread", [1.0, 8.0])
+def test_exact_attention_holds_f32_precision(hip, torch_cuda, S, spread):
+    """Head width 64, the f32 family on products of three-way bf16 splits:
+    2-norm error against float64 attention within 1e-6 a unit of the scores'
+    spread -- the part products left out are below 2^-26 of a product, an f32
+    rounding 2^-24, and a score's absolute error scales its weight (f32 MFMA
+    measured 8e-7 at spread 1); the fused dK / dV pass bit for bit the separate
+    ones."""
+    torch = torch_cuda
+    B, H, d = 2, 3, 64
+    print(f"exact attention S={S} spread={spread}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(S)
+    q, k, v, do = (torch.randn((B * S, H * d), device="cuda", generator=g) for _ in range(4))
+    q *= spread
+    o, dq, dk, dv, dk1, dv1 = (torch.full_like(q, float("nan")) for _ in range(6))
+    st = torch.empty((B * H * S, 4), device="cuda")
+    P = lambda t: t.data_ptr()  # noqa: E731
+    ctx = hip.Context(0)
+    ctx.use_torch_stream()
+    geo = (B, S, H, d)
+    ctx.call("seeai_attn_fwd", 0, P(q), P(k), P(v), P(o), P(st), *geo, None)
+    ctx.call("seeai_attn_dq", 0, P(q), P(k), P(v), P(do), P(st), P(dq), *geo)
+    ctx.call("seeai_attn_dkdv_f32", P(q), P(k), P(v), P(do), P(st), P(dk), P(dv), *geo)
+    ctx.call("seeai_attn_dk", 0, P(q), P(k), P(v), P(do), P(st), P(dk1), *geo)
+    ctx.call("seeai_attn_dv", 0, P(q), P(k), P(do), P(st), P(dv1), *geo)
+    torch.cuda.synchronize()
+    ctx.close()
+    assert torch.equal(dk, dk1) and torch.equal(dv, dv1)
+    split = lambda t: t.double().view(B, S, H, d).transpose(1, 2).contiguous()  # noqa: E731
+    Q, K, V, G = split(q), split(k), split(v), split(do)
+    i = torch.arange(S, device="cuda")
+    sc = (Q @ K.transpose(2, 3).contiguous() / 8.0).masked_fill(i[None] > i[:, None], -float("inf"))
+    p = torch.softmax(sc, dim=3)
+    dp = G @ V.transpose(2, 3).contiguous()
+    ds = p * (dp - (p * dp).sum(dim=3, keepdim=True)) / 8.0
+    want = {"o": p @ V, "dq": ds @ K, "dk": ds.transpose(2, 3).contiguous() @ Q,
+            "dv": p.transpose(2, 3).contiguous() @ G}
+    for name, got in [("o", o), ("dq", dq), ("dk", dk), ("dv", dv)]:
+        # one token: dS is exactly 0 in exact arithmetic, so dQ and dK compare to the products' size
+        size = max(float(want[name].norm()), float((G.norm() * K.norm()) if S == 1 else 0.0))
+        e = float((split(got) - want[name]).norm()) / size
+        assert e <= 1e-6 * spread, f"{name}: {e:.3g}"
+
+
 # --- optimizer -----------------------------------------------------------------------------
 
 @pytest.mark.parametrize("n", [1, 2048, 100003])
