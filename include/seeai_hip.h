@@ -204,8 +204,9 @@ typedef struct seeai_tile_policy {
   uint32_t relaxed_min_tiles_256; /* relaxed bf16 GEMM: 256x256 tiles from this many (default 256) */
   uint32_t relaxed_min_fill_256;  /* ... and when their last round over the CUs is at least
                                      this percent full (<= 100) */
-  uint32_t relaxed_nt_dma_min_k;  /* relaxed NT on rodata weights: the direct-to-LDS kernel from
-                                     this K, the register-staged one below (default 768) */
+  uint32_t relaxed_nt_dma_min_k;  /* relaxed NT on rodata weights: the direct-to-LDS kernel's
+                                     range fusions from this K (default 768); a value over 768
+                                     also keeps the register-staged kernel below it */
   uint32_t convert_wgs_per_cu;    /* workgroups per CU of the relaxed GEMMs' activation
                                      conversion (default 8, <= 64) */
   uint32_t exact_longk_first;     /* exact skinny long-K GEMM: 1 the two-pass form before the

@@ -436,7 +436,8 @@ int GemmBf16Dma(seeai_ctx* c, GemmArgs& a, const char* what) {
 // A GEMM launch with the workspace its kernel may use.
 int Gemm(seeai_ctx* c, GemmArgs& a, const char* what) {
   a.policy = &c->policy;
-  if (a.relaxed && c->allow_dma && Bf16DmaFits(a) && Immutable(c, a.B)) return GemmBf16Dma(c, a, what);
+  if (a.relaxed && c->allow_dma && Bf16DmaFitsAlone(a) && Immutable(c, a.B))
+    return GemmBf16Dma(c, a, what);
   if (const size_t bytes = a.relaxed ? 0 : GemmExactScratchBytes(a)) {
     void* ws;
     if (int rc = Scratch(c, bytes, &ws)) return rc;
@@ -2550,7 +2551,7 @@ int PresizeWorkspaces(seeai_ctx* c, const uint8_t* prog, uint64_t begin, uint64_
     if (!DecodeGemm(c, ins, &a)) continue;
     a.relaxed = (ins.flags & kFlagRelaxed) && c->allow_relaxed ? 1 : 0;
     a.policy = &c->policy;
-    if (a.relaxed && c->allow_dma && Bf16DmaFits(a) && Immutable(c, a.B)) {
+    if (a.relaxed && c->allow_dma && Bf16DmaFitsAlone(a) && Immutable(c, a.B)) {
       cvt = std::max(cvt, static_cast<size_t>(a.M * Bf16DmaKp(a.K) * 2));
       const auto key = std::make_tuple(a.B, a.layout, a.b_kind, static_cast<uint64_t>(a.N),
                                        static_cast<uint64_t>(a.K));

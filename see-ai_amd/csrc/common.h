@@ -350,8 +350,8 @@ struct TilePolicy {
   size_t relaxed_min_tiles_256 = 256;  // relaxed bf16 GEMM: 256 x 256 tiles from this many
   int relaxed_min_fill_256 = 0;        // ... and when their last round of tiles over
                                        // the CUs is at least this percent full
-  size_t relaxed_nt_dma_min_k = 768;   // relaxed NT: the direct-to-LDS kernel from this K
-                                       // (below it the register-staged bf16 kernel)
+  size_t relaxed_nt_dma_min_k = 768;   // relaxed NT: the direct-to-LDS kernel's range fusions
+                                       // from this K (over 768: the kernel itself)
   int convert_wgs_per_cu = 8;          // workgroups per CU of the activation conversion
   int exact_longk_first = 1;           // exact skinny long-K GEMM: 1 the two-pass workspace
                                        // form before the chain kernel, 2 the chain kernel first
@@ -419,7 +419,8 @@ size_t GemmExactScratchBytes(const GemmArgs& a);
 // (k_gemm_bf16dma.hip): A converted into a bf16 workspace [M, Kp] with its
 // scales, the weight's bf16 shadow [N, Kp] made once; Kp = K rounded up to 32.
 size_t Bf16DmaKp(size_t K);
-bool Bf16DmaFits(const GemmArgs& a);
+bool Bf16DmaFits(const GemmArgs& a);       // with the range fusions
+bool Bf16DmaFitsAlone(const GemmArgs& a);  // the product by itself
 // Whether the low-rank epilogue can join this product (N % 4 == 0, rank
 // operands 16-byte aligned, 1 <= lr_k <= kLowRankMaxK).
 bool Bf16DmaRowMaxFits(const GemmArgs& a);

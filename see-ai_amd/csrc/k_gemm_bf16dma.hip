@@ -204,26 +204,26 @@ GemmBf16DmaKernel(const __bf16* __restrict__ A, const __bf16* __restrict__ W, in
         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[slot][j], fa[slot][i], acc[i][j],
                                                             0, 0, 0);
   };
-  // The next k-step's TM + TN LDS reads spread one per MFMA; after the
-  // barrier the stage's loads take the last MFMA slots.
+  // The next k-step's TM + TN LDS reads spread over the MFMAs from the first;
+  // after the barrier the stage's loads take the last MFMA slots.
+  constexpr int kMfmas = TM * TN, kReads = TM + TN;
+  constexpr int kPerSlot = (kReads + kMfmas - 1) / kMfmas;
   auto interleave = [&]() {
 #pragma unroll
-    for (int s = 0; s < TM + TN; ++s) {
+    for (int s = 0; s < kMfmas; ++s) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      if (s * kPerSlot < kReads) __builtin_amdgcn_sched_group_barrier(0x100, kPerSlot, 0);
     }
-#pragma unroll
-    for (int s = TM + TN; s < TM * TN; ++s) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
   };
   auto interleave_loads = [&]() {
 #pragma unroll
-    for (int s = 0; s < TM * TN; ++s) {
+    for (int s = 0; s < kMfmas; ++s) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      if (s < TM + TN) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      if (s >= TM * TN - kPerStage) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+      if (s * kPerSlot < kReads) __builtin_amdgcn_sched_group_barrier(0x100, kPerSlot, 0);
+      if (kMfmas >= kPerStage && s >= kMfmas - kPerStage)
+        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
     }
   };
-  static_assert(TM * TN >= TM + TN && TM * TN >= kPerStage, "MFMA slots for the reads and loads");
 
   // Every iteration loads one stage; past the last the loads repeat it (in
   // bounds, into a buffer no later stage uses), so the stages in flight at
@@ -726,18 +726,38 @@ hipError_t Launch(const __bf16* A, const __bf16* W, size_t Kp, const GemmArgs& g
 
 size_t Bf16DmaKp(size_t K) { return (K + 31) / 32 * 32; }
 
-bool Bf16DmaFits(const GemmArgs& a) {
+namespace {
+constexpr size_t kMinK = 64;           // every layout
+constexpr size_t kNtDefaultMinK = 768;  // relaxed_nt_dma_min_k's default
+bool DmaFits(const GemmArgs& a, size_t nt_min_k) {
   if (!a.relaxed || a.layout > 1 || a.b_kind > 2) return false;
-  if (a.M < 128 || a.N < 128 || a.K < 64) return false;
-  // NT below the tile policy's relaxed_nt_dma_min_k runs the
-  // register-staged kernel (at short K the conversion pass can cost more
-  // than it saves).
-  if (a.layout == 1 && a.K < (a.policy ? a.policy->relaxed_nt_dma_min_k : 768)) return false;
+  if (a.M < 128 || a.N < 128 || a.K < kMinK) return false;
+  if (a.layout == 1 && a.K < nt_min_k) return false;
   const size_t Kp = Bf16DmaKp(a.K);
   // 32-bit buffer offsets within a tile and int tile indices.
   if (Kp * 2 * 256 >= (size_t{1} << 31) || a.M >= (size_t{1} << 30) || a.N >= (size_t{1} << 30))
     return false;
   return ((a.M + 127) / 128) * ((a.N + 127) / 128) < (size_t{1} << 31);
+}
+size_t NtMinK(const GemmArgs& a) {
+  return a.policy ? a.policy->relaxed_nt_dma_min_k : kNtDefaultMinK;
+}
+}  // namespace
+
+// NT products join the range fusions from the tile policy's
+// relaxed_nt_dma_min_k.
+bool Bf16DmaFits(const GemmArgs& a) { return DmaFits(a, NtMinK(a)); }
+
+// Launched by itself an NT product takes this kernel from K = 64: its smaller
+// tiles pay for the conversion pass at every K.  Register-staged / this with
+// the pass, us, f32 weights: 128 x 128 x 64 10.8 / 7.3, 2048 x 1024 x 256 16.0
+// / 8.9, 8192 x 256 x 256 18.3 / 10.5, 8192 x 2048 x 512 63 / 35, 8192 x 32000
+// x 64 568 / 280; int8 weights 12.9 / 7.4, 20.7 / 8.9, 23.0 / 10.5, 93 / 35,
+// 614 / 283.  A policy that raises its threshold over the default keeps the
+// register-staged kernel below it.
+bool Bf16DmaFitsAlone(const GemmArgs& a) {
+  const size_t nt = NtMinK(a);
+  return DmaFits(a, nt <= kNtDefaultMinK ? kMinK : nt);
 }
 
 // The partial row maxima ride the epilogue that stores from registers: no
@@ -820,8 +840,8 @@ hipError_t LaunchWeightShadow(const GemmArgs& a, void* out, hipStream_t s) {
 // policy's relaxed_min_tiles_256 of them (default 256: one per CU) and they
 // fill the CUs' last round of tiles to at least relaxed_min_fill_256 percent
 // (384 tiles on 256 CUs: 75 %); otherwise
-// 128 x 128 (four waves of 64 x 64).  Both accumulate each output over k in
-// the same 16-deep MFMA steps: the same bits.
+// 128 x 128 (four waves of 64 x 64), or 64 x 64 for few of them.  All
+// accumulate each output over k in the same 16-deep MFMA steps: the same bits.
 hipError_t LaunchGemmBf16Dma(const void* A, const void* W, const GemmArgs& a, hipStream_t s) {
   // The partial row maxima and (with no low-rank term) C's bf16 copy ride
   // the epilogue that stores from registers.
@@ -852,6 +872,23 @@ hipError_t LaunchGemmBf16Dma(const void* A, const void* W, const GemmArgs& a, hi
   if (a.N >= 192 && !a.row_max_part &&
       (mode == 3 || (mode == 1 && (c192 < c128 || (c192 == c128 && r192 <= r128)))))
     return Launch<128, 192, 2, 2, 3>(Ab, Wb, Kp, a, s);
+  // 64 x 64 (four waves of 32 x 32) where 128 x 128 tiles would leave half the
+  // CUs without one: a tile's k loop is bound by the latency of its loads
+  // (0.33 us per 32-deep stage on 128 x 128), so more, smaller tiles win until
+  // there are two per CU.  Up to one 64 x 64 tile per CU eight stages hide
+  // more of it.  With the conversion of A, us, 128 x 128 / 64 x 64 with 4
+  // stages / with 8: NT K = 2048, 16 tiles of 128 x 128 21.6 / 17.4 / 13.6,
+  // 64 23.5 / 18.7 / 15.3, 96 25.7 / 22.5 / 24.0, 128 26.0 / 24.2 / 26.3, 160
+  // 26.9 / 33.1 / 34.0; K = 256 8.6 / 7.2 / 7.3, 9.0 / 7.3 / 7.2, 9.6 / 8.2 /
+  // 8.7, 9.7 / 8.9 / 9.5, 10.3 / 10.2 / 11.5.  Eight stages of 128 x 128 gain
+  // nothing (21.3, 22.9, 25.0), 128 x 64 less than 64 x 64 up to 64 tiles.
+  // (No instance for the partial row maxima, which need 64-column wave
+  // slices.)
+  if (!a.row_max_part && 2 * t128 <= cus) {
+    const size_t t64 = ((a.M + 63) / 64) * ((a.N + 63) / 64);
+    if (t64 <= cus) return Launch<64, 64, 2, 2, 8>(Ab, Wb, Kp, a, s);
+    return Launch<64, 64, 2, 2, 4>(Ab, Wb, Kp, a, s);
+  }
   return Launch<128, 128, 2, 2, 4>(Ab, Wb, Kp, a, s);
 }
 

@@ -45,7 +45,8 @@ FIELDS = {
                              "relaxed bf16 GEMM: 256x256 tiles only when their last round over "
                              "the CUs is at least this percent full"),
     "relaxed_nt_dma_min_k": (768, ("range", 64, 1 << 30),
-                             "relaxed NT on rodata weights: the direct-to-LDS kernel from this K"),
+                             "relaxed NT on rodata weights: the direct-to-LDS kernel's range fusions "
+                             "from this K (over 768: the kernel itself)"),
     "convert_wgs_per_cu": (8, ("range", 1, 64),
                            "workgroups per CU of the relaxed GEMMs' activation conversion"),
     "exact_longk_first": (1, ("choice", 1, 2),

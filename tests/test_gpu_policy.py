@@ -179,3 +179,56 @@ def test_relaxed_nt_kernel_arms_are_bitwise_equal(hip, torch_cuda, kind):
         be.ctx.close()
     assert np.isfinite(outs[0]).all()
     assert bits_equal(outs[1], outs[0])
+
+
+@pytest.mark.parametrize("kind", ["f32", "q8"])
+@pytest.mark.parametrize("nt", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(128, 128, 64), (129, 190, 65), (200, 193, 320), (1000, 130, 96),
+                                   (1300, 1281, 128), (1984, 1024, 2080)])
+def test_relaxed_small_tiles_are_bitwise_the_large_ones(hip, torch_cuda, M, N, K, nt, kind):
+    """A relaxed product of few output tiles runs 64 x 64 tiles (eight load
+    stages up to one per CU, else four); the same rows at the head of a
+    product of enough rows for 128 x 128 tiles have the same bits, every
+    output being the same k-order of MFMA steps."""
+    from tests.plan_ops import ins
+    from tests.arena import f32_bits
+    print(f"policy: small tiles {kind} nt {nt} {M}x{N}x{K}", flush=True)
+    big = 128 * (1 + 129 // ((N + 127) // 128)) + 1
+    assert ((big + 127) // 128) * ((N + 127) // 128) > 128 >= ((M + 127) // 128) * ((N + 127) // 128)
+    big = max(big, M)
+    r = rng(M + N + K + nt)
+    A = r.standard_normal((big, K)).astype(np.float32)
+    shape = (N, K) if nt else (K, N)
+    if kind == "q8":
+        W = r.integers(-127, 128, shape).astype(np.int8)
+    else:
+        W = (r.standard_normal(shape) * 0.02).astype(np.float32)
+    ks = r.uniform(1e-3, 5e-2, K if nt else N).astype(np.float32)
+    ar = Arena()
+    a = ar.add("A", A)
+    w, s = ar.add("W", W, rodata=True), ar.add("ks", ks, rodata=True)
+    outs = [ar.empty("Cs", (M, N)), ar.empty("Cl", (big, N))]
+    arena, ro = ar.images()
+    be = hip.HipBackend(0)
+    be.Bind(arena.tobytes(), arena.nbytes, ro.tobytes())
+    for o, rows in zip(outs, (M, big)):
+        if kind == "q8":
+            be.Execute(ins(30 if nt else 29, [a, w, o, s], [rows, N, K], flags=(1 << 5) | (1 << 4)))
+        else:
+            be.Execute(ins(2 if nt else 1, [a, w, o], [rows, N, K], flags=1 << 5,
+                           imm=f32_bits(0.37)))
+    be.Flush()
+    got = np.frombuffer(be.Download(0, arena.nbytes), np.uint8)
+    small, large = ar.get(got, "Cs"), ar.get(got, "Cl")
+    be.ctx.close()
+    assert np.isfinite(small).all()
+    assert bits_equal(small, large[:M])
+    scale = ks if kind == "q8" else np.float32(1)
+    Wd, Ad = W.astype(np.float64), A[:M].astype(np.float64)
+    if kind == "q8":
+        Wd = Wd * scale if nt else Wd * scale[None, :]
+    want = Ad @ (Wd.T if nt else Wd) * (1 if kind == "q8" else 0.37)
+    bound = np.abs(Ad) @ (np.abs(Wd).T if nt else np.abs(Wd))
+    # Operands rounded once to bf16 (2^-8 each, q8 weights exactly held) and
+    # the f32 sum of K terms.
+    assert (np.abs(small - want) <= bound * (2 * 2.0 ** -8 + K * 2.0 ** -23)).all()
