@@ -1633,15 +1633,18 @@ bool Fold(const GemmArgs& a) {
 }
 
 // NN with a narrow f32 B -- the LoRA products t = X A, N = 8 or 16 -- over
-// many rows and K past the panel kernel's: role-split folds of 32 x 8 or
+// many rows: role-split folds of 32 x 8 or
 // 16 x 16 output blocks, four outputs per folder lane, 128-deep chunks (two
 // workgroups' LDS per CU).  C4's 8192 x 8 x 768: 17.8 us on the chain
 // kernel -> 8.0; C5's 8192 x 16 x 2048: 37.9 on the 8 x 16 fold -> 29-30
-// (one box, bitwise the same sums).
+// (one box, bitwise the same sums).  Short K too, against the panel: 2048 x 8
+// x 128 6.0 -> 4.7, 4096 x 8 x 320 12.2 -> 5.9, 6272 x 16 x 320 12.9 -> 10.0,
+// 4096 x 16 x 512 18.2 -> 6.2.
 bool FoldNarrowNN(const GemmArgs& a) {
   const auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   return a.layout == 0 && a.b_kind == 0 && (a.N == 8 || a.N == 16) &&
-         a.K > static_cast<size_t>(kPanelK) && a.K % 4 == 0 && a.M % 32 == 0 && a.M >= 4096 &&
+         a.K >= 128 && a.K % 4 == 0 && a.M % 32 == 0 &&
+         a.M >= (a.K > static_cast<size_t>(kPanelK) ? 4096 : 2048) &&
          a.M / 16 <= 65535 && a.K * a.M < (size_t{1} << 31) && al16(a.A) && al16(a.B) &&
          !a.a_k_scale;
 }
@@ -1703,10 +1706,12 @@ hipError_t LaunchFold(const GemmArgs& a, hipStream_t s) {
 // reduction it carries: under 512 tiles of 64 x 64 and K above the panel.
 // NT's tiled kernel (32 x 64 blocks, eight chains an output) takes over
 // earlier: 512 x 2560 x 704, 320 blocks of 64 x 64, 136 us here and 115 there;
-// 512 x 768 x 768, 96 blocks, 33 and 59.
+// 512 x 768 x 768, 96 blocks, 33 and 59.  (Not where a block's columns or rows
+// are mostly past the output.)
 bool Chain(const GemmArgs& a) {
   const size_t tiles = ((a.M + 63) / 64) * ((a.N + 63) / 64);
-  return a.K > static_cast<size_t>(kPanelK) && tiles < (a.layout == 1 ? 320 : 512);
+  const bool whole = a.M >= 64 && a.N >= 64;
+  return a.K > static_cast<size_t>(kPanelK) && tiles < (a.layout == 1 && whole ? 320 : 512);
 }
 
 template <int kLayout, int kBKind, int BM, int BN>
@@ -1721,11 +1726,13 @@ hipError_t LaunchChain(const GemmArgs& a, hipStream_t s) {
 
 bool LongK(const GemmArgs& a) { return a.layout != 1 && a.M * a.N <= 16384 && a.K >= 1024; }
 
-// NT over at most 16 outputs per row, enough rows to fill the machine and a
-// long K, with 16-byte rows of A: the k-lane kernel.
+// NT over at most 16 outputs per row, enough rows to fill the machine (below,
+// NTLanes runs), with 16-byte rows of A: the k-lane kernel.  Against the panel,
+// us: 2048 x 8 x 64 4.7 / 4.6 here, x 128 7.3 / 4.6, x 256 12.5 / 5.1, x 512
+// 23.0 / 7.6; 6272 x 16 x 320 16.3 / 8.2.
 bool KLane(const GemmArgs& a) {
   return a.layout == 1 && a.b_kind == 0 && !a.a_k_scale && a.N <= 16 && a.M >= 2048 &&
-         a.K >= 256 && a.K % 4 == 0 && (reinterpret_cast<uintptr_t>(a.A) & 15) == 0 &&
+         a.K >= 64 && a.K % 4 == 0 && (reinterpret_cast<uintptr_t>(a.A) & 15) == 0 &&
          a.M * a.K < (size_t{1} << 40);
 }
 
@@ -1781,8 +1788,13 @@ size_t Tiles64(const GemmArgs& a) { return ((a.M + 63) / 64) * ((a.N + 63) / 64)
 // x 512, 128 blocks of 64 x 64, 44 us against 27), and not so many that the
 // 64 x 64 tiles' lower LDS traffic counts (2048 x 32000 x 768: 2339 us
 // against 2096; 8192 x 768 x 768, 1536 blocks: 225 / 222).
+// Past the panel's K the chain kernel is what it replaces, whose time goes with
+// the outputs, so a narrow product needs as many of them (N = 32, K = 768,
+// here / chain: M = 12800 64 / 51, 25600 66 / 83; K = 2048 164 / 130, 167 /
+// 212).
 bool Tile(const GemmArgs& a) {
-  return TileFits(a) && a.M >= kTile && a.N >= kTile && Tiles64(a) >= 200 && Tiles64(a) < 1024;
+  return TileFits(a) && a.M >= kTile && a.N >= kTile && Tiles64(a) >= 200 && Tiles64(a) < 1024 &&
+         (a.K <= static_cast<size_t>(kPanelK) || a.M * a.N >= size_t{200} * 64 * 64);
 }
 
 template <int kLayout, int kBKind>
@@ -1798,9 +1810,10 @@ hipError_t LaunchTile(const GemmArgs& a, hipStream_t s) {
 // too few rows for them.  us, old route / rows: 1024 x 512 x 512 74 (panel) /
 // 28, 1024 x 256 x 256 15 / 10.5, 2048 x 128 x 128 9.3 / 7.0, 512 x 768 x 768
 // 39 (chain) / 33, 8 x 32000 x 768 40 / 31; but 256 x 768 x 768 (48 blocks) 21
-// / 26, 64 x 256 x 256 (4) 8.8 / 9.3.
+// / 26, 64 x 256 x 256 (4) 8.8 / 9.3.  Not over long K, where the chain kernel's
+// LDS serves it better: 5120 x 64 x 768 35 / 30, x 2048 88 / 108.
 bool Rows(const GemmArgs& a) {
-  if (a.layout != 0 || a.K < 4 || a.K % 4 != 0 || a.alpha_a != 1.0f || a.a_k_scale || a.N < 64)
+  if (a.layout != 0 || a.K < 4 || a.K > 1024 || a.K % 4 != 0 || a.alpha_a != 1.0f || a.a_k_scale || a.N < 64)
     return false;
   const size_t t = Tiles64(a);
   return t >= (a.K <= static_cast<size_t>(kPanelK) ? 32u : 80u) && (t < 200 || a.M < kTile);
@@ -1820,10 +1833,18 @@ hipError_t LaunchRows(const GemmArgs& a, hipStream_t s) {
 // outputs that fill the machine with one lane each, the tiled kernel's
 // register blocks are several times faster (us, panel / tiled: 1024 x 512 x
 // 512 NT, 128 blocks of 64 x 64, 92 / 41; 8192 x 2048 x 512 NN 2760 / 390, NT
-// 3382 / 660; but 1024 x 256 x 256 NT, 64 blocks, 17 / 22).
+// 3382 / 660; but 1024 x 256 x 256 NT, 64 blocks, 17 / 22).  Fewer columns (or
+// rows) than a block leave most of its lanes idle, so there the panel's own 16
+// x 16 blocks count: NN 8192 x 12 x 256, 512 of them, 11 / 31; 8192 x 24 x 512
+// (1024) 47 / 58; 16384 x 24 (2048) 14 / 18 at K = 128, 32 / 32 at 256, 93 / 59
+// at 512.  NT's rows of eight lanes gain less from it: 8192 x 24 (1024) 17 /
+// 22 at K = 256, 56 / 40 at 512; 8192 x 12 x 512 (512) 24 / 40.
 bool Panel(const GemmArgs& a) {
-  return a.K > 0 && a.K <= static_cast<size_t>(kPanelK) && (a.M + 15) / 16 <= 65535 &&
-         (a.M <= 16 || Tiles64(a) < 100);
+  if (a.K == 0 || a.K > static_cast<size_t>(kPanelK) || (a.M + 15) / 16 > 65535) return false;
+  if (a.M <= 16 || Tiles64(a) < 100) return true;
+  const size_t blocks = ((a.M + 15) / 16) * ((a.N + 15) / 16);
+  if (a.layout == 1) return blocks <= 1024 && blocks * a.K <= 327680;
+  return blocks <= (a.K <= 256 ? 2048 : 1024);
 }
 
 template <int kLayout, int kBKind>
@@ -1849,16 +1870,8 @@ hipError_t Run(const GemmArgs& a, hipStream_t s) {
     const bool fold = Fold(a) || FoldNarrowNN(a) || (LongK(a) && a.scratch && LongKFirst(a));
     if (Tile(a) && !fold) return LaunchTile<kLayout, kBKind>(a, s);
   }
-  if (Panel(a)) {
-    const dim3 grid(static_cast<unsigned>((a.N + 15) / 16), static_cast<unsigned>((a.M + 15) / 16));
-    const size_t lds = 2 * 16 * a.K * sizeof(float);
-    hipLaunchKernelGGL((GemmPanelKernel<kLayout, kBKind>), grid, dim3(kThreads), lds, s, a);
-    return hipGetLastError();
-  }
   if constexpr (kLayout == 0 && kBKind == 0)
     if (FoldNarrowNN(a)) return LaunchFoldNarrowNN(a, s);
-  if constexpr (kLayout != 1 && kBKind == 0)
-    if (Fold(a)) return LaunchFold<kLayout>(a, s);
   if constexpr (kLayout == 1 && kBKind == 0)
     if (KLane(a)) {
       if (a.N <= 8) {
@@ -1870,6 +1883,14 @@ hipError_t Run(const GemmArgs& a, hipStream_t s) {
       }
       return hipGetLastError();
     }
+  if (Panel(a)) {
+    const dim3 grid(static_cast<unsigned>((a.N + 15) / 16), static_cast<unsigned>((a.M + 15) / 16));
+    const size_t lds = 2 * 16 * a.K * sizeof(float);
+    hipLaunchKernelGGL((GemmPanelKernel<kLayout, kBKind>), grid, dim3(kThreads), lds, s, a);
+    return hipGetLastError();
+  }
+  if constexpr (kLayout != 1 && kBKind == 0)
+    if (Fold(a)) return LaunchFold<kLayout>(a, s);
   if (Chain(a) && !(kLayout != 1 && LongK(a) && a.scratch && LongKFirst(a))) {
     if (a.N <= 8) return LaunchChain<kLayout, kBKind, 32, 8>(a, s);
     if (a.M <= 8) return LaunchChain<kLayout, kBKind, 8, 32>(a, s);

@@ -293,6 +293,16 @@ def test_gemm_narrow_weights_on_tiles_and_rows(hip, orc, backend, M, N, K):
     test_gemm_narrow_weights(hip, orc, backend, M, N, K)
 
 
+# Narrow products of many rows: the k-lane kernel (NT) and the narrow fold (NN)
+# at short K, below and past their smallest; the panel past 100 blocks of 64 x
+# 64; few 32 x 32 tiles past the panel's K (the chain kernel).
+@pytest.mark.parametrize("M,N,K", [(2048, 8, 64), (2080, 8, 132), (2080, 16, 388), (2047, 8, 128),
+                                   (2049, 3, 68), (6432, 12, 96), (6500, 24, 260),
+                                   (12800, 32, 516)])
+def test_gemm_f32_over_many_narrow_rows(hip, orc, backend, M, N, K):
+    test_gemm_f32_family(hip, orc, backend, M, N, K, False)
+
+
 # --- elementwise / activation / normalization -------------------------------------
 
 def test_elementwise_family(hip, orc, backend):
