@@ -105,9 +105,9 @@ ORACLE_ONLY = {
 
 
 def build(ref: bool = True) -> None:
-    """Compile liboracle.so (and _ref where /root/reference exists)."""
+    """Compile liboracle.so (and _ref where /root/reference holds its sources)."""
     targets = ["oracle"]
-    if ref and os.path.isdir(REFERENCE_ROOT):
+    if ref and os.path.isfile(os.path.join(REFERENCE_ROOT, "runtime", "executor", "gemm.cc")):
         targets.append("ref")
     subprocess.run(["make", "-s", "-C", HERE, *targets], check=True)
 
