@@ -34,6 +34,11 @@
 // workgroups share a CU and one multiplies while the other stages.  Tiles, fragments and the
 // transposed score layout are k_attn16.hip's.
 //
+// An infinity, a NaN, or a float past the largest bf16 (3.3895e38) has no such
+// parts: its last one is NaN, and with it every sum it joins.  A wave whose sums
+// come out NaN forms its rows again in plain f32 (PlainFwd, PlainDQ, PlainDKDV),
+// so they hold what f32 arithmetic gives and only where it does.
+//
 // Every output element has one writer and every sum a fixed order; dK and dV
 // are one template, so the fused pass has the separate passes' bits.
 #include "attn_tile.h"
@@ -63,16 +68,13 @@ __device__ __forceinline__ void UnitOf3(int nb, int& bh, int& rank) {
 struct Parts {
   bf16x8 p[3];  // h, m, l
 };
-// Eight floats in their parts.  kFinite: no infinities among them; otherwise
-// an infinity is its own first part and the rest is zero.
-template <bool kFinite>
+// Eight floats in their parts.
 __device__ __forceinline__ Parts Split(const float (&x)[8]) {
   Parts r;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     r.p[0][i] = static_cast<__bf16>(x[i]);
-    float rest = x[i] - static_cast<float>(r.p[0][i]);
-    if (!kFinite) rest = rest == rest ? rest : 0.0f;
+    const float rest = x[i] - static_cast<float>(r.p[0][i]);
     r.p[1][i] = static_cast<__bf16>(rest);
     r.p[2][i] = static_cast<__bf16>(rest - static_cast<float>(r.p[1][i]));
   }
@@ -112,7 +114,7 @@ struct Block3 {
       const int row = e * 32 + threadIdx.x / 8, ch = threadIdx.x % 8;
       const float x[8] = {r[2 * e].x,     r[2 * e].y,     r[2 * e].z,     r[2 * e].w,
                           r[2 * e + 1].x, r[2 * e + 1].y, r[2 * e + 1].z, r[2 * e + 1].w};
-      const Parts s = Split<false>(x);
+      const Parts s = Split(x);
       const int at = ch / 4 * kHalf + row * 64 + Phys(row, ch % 4) * 16;
 #pragma unroll
       for (int p = 0; p < 3; ++p) *reinterpret_cast<bf16x8*>(t.part[p] + at) = s.p[p];
@@ -127,7 +129,7 @@ __device__ __forceinline__ void OwnParts(const float* __restrict__ row, int lane
     const float* p = row + 16 * s + 8 * (lane / 32);
     const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
     const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-    f[s] = Split<false>(x);
+    f[s] = Split(x);
   }
 }
 __device__ __forceinline__ Parts RowParts(const Tile3& t, const FragOffsets& fo, int row0, int s) {
@@ -156,7 +158,7 @@ __device__ __forceinline__ void Accum3(const Tile3& t, const FragOffsets& fo, in
   for (int h = 0; h < 2; ++h) {
     const float x[8] = {w[8 * h],     w[8 * h + 1], w[8 * h + 2], w[8 * h + 3],
                         w[8 * h + 4], w[8 * h + 5], w[8 * h + 6], w[8 * h + 7]};
-    b[h] = Split<true>(x);
+    b[h] = Split(x);
   }
 #pragma unroll
   for (int dt = 0; dt < 2; ++dt) {
@@ -190,6 +192,112 @@ __device__ __forceinline__ void KeyBlocks(int start, int i0, int S, int& first, 
   __syncthreads();
   first = min(min(lo[0], lo[1]), min(lo[2], lo[3])) / kBlkRows;
   count = min(i0 + kRowsWG - 1, S - 1) / kBlkRows - first + 1;
+}
+
+// ---------------------------------------------------------------------------
+// The same rows in plain f32, a multiply-add at a time, each over the rows it
+// sees and no other: for the waves whose sums came out NaN.  Two lanes a row
+// (lane % 32), 32 of the 64 dims each; slow and rare.
+// ---------------------------------------------------------------------------
+struct Half {  // a lane's 32 dims of a row
+  float x[32];
+  __device__ __forceinline__ explicit Half(const float* row, int g) {
+#pragma unroll
+    for (int e = 0; e < 32; e += 4) {
+      const float4 v = *reinterpret_cast<const float4*>(row + 32 * g + e);
+      x[e] = v.x, x[e + 1] = v.y, x[e + 2] = v.z, x[e + 3] = v.w;
+    }
+  }
+  __device__ __forceinline__ Half() {
+#pragma unroll
+    for (int e = 0; e < 32; ++e) x[e] = 0.0f;
+  }
+  // this += w r
+  __device__ __forceinline__ void Add(float w, const Half& r) {
+#pragma unroll
+    for (int e = 0; e < 32; ++e) x[e] = __builtin_fmaf(w, r.x[e], x[e]);
+  }
+  __device__ __forceinline__ void Store(float* row, int g, float scale) const {
+#pragma unroll
+    for (int e = 0; e < 32; e += 4)
+      *reinterpret_cast<float4*>(row + 32 * g + e) =
+          make_float4(x[e] * scale, x[e + 1] * scale, x[e + 2] * scale, x[e + 3] * scale);
+  }
+};
+// The rows' dot over both lanes, the same in both.
+__device__ __forceinline__ float Dot(const Half& a, const Half& b) {
+  float s = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 32; ++e) s = __builtin_fmaf(a.x[e], b.x[e], s);
+  return SwapSum(s);
+}
+
+// Whether any of the wave's sums is NaN (wave-uniform).
+__device__ __forceinline__ bool AnyNaN(const v16f (&acc)[2], bool nan = false) {
+#pragma unroll
+  for (int r = 0; r < 16; ++r) nan |= __builtin_isunordered(acc[0][r], acc[1][r]);
+  return __ballot(nan) != 0;
+}
+
+// Query i's keys start .. i; every lane walks the wave's range first .. last.
+__device__ __forceinline__ void PlainFwd(const float* q_row, const float* k, const float* v,
+                                         size_t ld, int i, int start, int first, int last, int g,
+                                         Half& acc, float& m, float& l) {
+  const Half q(q_row, g);
+  m = -INFINITY, l = 0.0f;
+#pragma unroll 1
+  for (int j = first; j <= last; ++j) {
+    const float s = Dot(Half(k + static_cast<size_t>(j) * ld, g), q) * kIsd;
+    if (j < start || j > i) continue;
+    const float mn = fmaxf(m, s), alpha = m == -INFINITY ? 0.0f : expf(m - mn);
+    const float p = s == -INFINITY ? 0.0f : expf(s - mn);
+    l = l * alpha + p;
+    m = mn;
+#pragma unroll
+    for (int e = 0; e < 32; ++e) acc.x[e] *= alpha;
+    acc.Add(p, Half(v + static_cast<size_t>(j) * ld, g));
+  }
+}
+
+__device__ __forceinline__ void PlainDQ(const float* q_row, const float* d_row, const float* k,
+                                        const float* v, size_t ld, float m, float inv, int i,
+                                        int start, int first, int last, int g, Half& acc,
+                                        float& delta) {
+  const Half q(q_row, g), d(d_row, g);
+  double sum = 0.0;
+#pragma unroll 1
+  for (int pass = 0; pass < 2; ++pass) {
+    delta = static_cast<float>(sum);
+#pragma unroll 1
+    for (int j = first; j <= last; ++j) {
+      const Half kj(k + static_cast<size_t>(j) * ld, g);
+      const float s = Dot(kj, q), dp = Dot(Half(v + static_cast<size_t>(j) * ld, g), d);
+      if (j < start || j > i) continue;
+      const float p = expf(s * kIsd - m) * inv;
+      if (pass == 0)
+        sum += static_cast<double>(dp) * p;
+      else
+        acc.Add((p * (dp - delta)) * kIsd, kj);
+    }
+  }
+}
+
+// Key j's queries first .. S - 1 that see it.
+template <bool kDK, bool kDV>
+__device__ __forceinline__ void PlainDKDV(const float* k_row, const float* v_row, const float* q,
+                                          const float* dout, size_t ld, const float4* st, int j,
+                                          int first, int S, int g, Half& dk, Half& dv) {
+  const Half k(k_row, g), v(kDK ? v_row : k_row, g);
+#pragma unroll 1
+  for (int i = first; i < S; ++i) {
+    const float4 t = st[i];
+    const Half qi(q + static_cast<size_t>(i) * ld, g), di(dout + static_cast<size_t>(i) * ld, g);
+    const float s = Dot(qi, k), dp = kDK ? Dot(di, v) : 0.0f;
+    if (j > i || j < StartOf(t.w, i)) continue;
+    const float p = expf(s * kIsd - t.x) * t.y;
+    if (kDV) dv.Add(p, di);
+    if (kDK) dk.Add((p * (dp - t.z)) * kIsd, qi);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -281,9 +389,18 @@ Attn3Fwd(const float* __restrict__ q, const float* __restrict__ k, const float* 
     for (int t = 0; t < 2; ++t)
       if (j0 + 32 * t <= wave_last) Accum3(vt, fo, 32 * t, p[t], acc);
   }
+  l = SwapSum(l);
+  const size_t at = base + static_cast<size_t>(ic) * ld;
+  const bool plain = AnyNaN(acc, l != l);
+  Half row;
+  if (plain)
+    PlainFwd(q + at, k + base, v + base, ld, ic, start, WaveMinI(start), wave_last, g, row, m, l);
   if (i >= S) return;
-  const float inv = 1.0f / SwapSum(l);
-  StoreRow(o + base + static_cast<size_t>(i) * ld, g, acc, inv);
+  const float inv = 1.0f / l;
+  if (plain)
+    row.Store(o + at, g, inv);
+  else
+    StoreRow(o + at, g, acc, inv);
   if (g == 0)
     *reinterpret_cast<float4*>(stats + (static_cast<size_t>(bh) * S + i) * 4) =
         make_float4(m, inv, 0.0f, static_cast<float>(start));
@@ -361,12 +478,21 @@ Attn3DQ(const float* __restrict__ q, const float* __restrict__ k, const float* _
       Accum3(kt, fo, 32 * t, p, acc_p);
     }
   }
-  const float delta = static_cast<float>(dsum + __shfl_xor(dsum, 32, kWave));
+  float delta = static_cast<float>(dsum + __shfl_xor(dsum, 32, kWave));
   v16f acc[2];
 #pragma unroll
   for (int dt = 0; dt < 2; ++dt) acc[dt] = (acc_d[dt] - delta * acc_p[dt]) * kIsd;
+  const size_t at = base + static_cast<size_t>(ic) * ld;
+  const bool plain = AnyNaN(acc, delta != delta);
+  Half row;
+  if (plain)
+    PlainDQ(q + at, dout + at, k + base, v + base, ld, st.x, st.y, ic, start, WaveMinI(start),
+            wave_last, g, row, delta);
   if (i >= S) return;
-  StoreRow(dq + base + static_cast<size_t>(i) * ld, g, acc, 1.0f);
+  if (plain)
+    row.Store(dq + at, g, 1.0f);
+  else
+    StoreRow(dq + at, g, acc, 1.0f);
   if (g == 0) stats[(static_cast<size_t>(bh) * S + i) * 4 + 2] = delta;
 }
 
@@ -457,10 +583,21 @@ Attn3DKDV(const float* __restrict__ q, const float* __restrict__ k, const float*
       }
     }
   }
+  const size_t at = base + static_cast<size_t>(jc) * ld;
+  const bool plain_k = kDK && AnyNaN(acc_k), plain_v = kDV && AnyNaN(acc_v);
+  Half row_k, row_v;
+  if (plain_k || plain_v)
+    PlainDKDV<kDK, kDV>(k + at, v + (kDK ? at : 0), q + base, dout + base, ld, st, jc, jw, S, g,
+                        row_k, row_v);
   if (j >= S) return;
-  const size_t at = base + static_cast<size_t>(j) * ld;
-  if constexpr (kDK) StoreRow(dk + at, g, acc_k, 1.0f);
-  if constexpr (kDV) StoreRow(dv + at, g, acc_v, 1.0f);
+  if (plain_k)
+    row_k.Store(dk + at, g, 1.0f);
+  else if constexpr (kDK)
+    StoreRow(dk + at, g, acc_k, 1.0f);
+  if (plain_v)
+    row_v.Store(dv + at, g, 1.0f);
+  else if constexpr (kDV)
+    StoreRow(dv + at, g, acc_v, 1.0f);
 }
 
 dim3 GridOf(size_t B, size_t S, size_t H) {

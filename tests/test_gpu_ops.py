@@ -689,6 +689,115 @@ def test_exact_attention_holds_f32_precision(hip, torch_cuda, S, spread):
         assert e <= 1e-6 * spread, f"{name}: {e:.3g}"
 
 
+def _exact_attention(hip, torch, q, k, v, do, B, S, H, starts=None):
+    """The f32 family at head width 64 on host arrays of [B*S, H*64] floats:
+    o, dq, dk, dv as [B, H, S, 64] float64 arrays."""
+    d = 64
+    q, k, v, do = (torch.from_numpy(np.ascontiguousarray(t, np.float32)).cuda() for t in (q, k, v, do))
+    o, dq, dk, dv, dk1, dv1 = (torch.full_like(q, 12345.0) for _ in range(6))
+    st = torch.empty((B * H * S, 4), device="cuda")
+    if starts is not None:
+        starts = torch.from_numpy(starts).cuda()
+    P = lambda t: t.data_ptr()  # noqa: E731
+    ctx = hip.Context(0)
+    ctx.use_torch_stream()
+    geo = (B, S, H, d)
+    ctx.call("seeai_attn_fwd", 0, P(q), P(k), P(v), P(o), P(st), *geo,
+             P(starts) if starts is not None else None)
+    ctx.call("seeai_attn_dq", 0, P(q), P(k), P(v), P(do), P(st), P(dq), *geo)
+    ctx.call("seeai_attn_dkdv_f32", P(q), P(k), P(v), P(do), P(st), P(dk), P(dv), *geo)
+    ctx.call("seeai_attn_dk", 0, P(q), P(k), P(v), P(do), P(st), P(dk1), *geo)
+    ctx.call("seeai_attn_dv", 0, P(q), P(k), P(do), P(st), P(dv1), *geo)
+    torch.cuda.synchronize()
+    ctx.close()
+    for fused, alone in ((dk, dk1), (dv, dv1)):  # the same bits
+        assert np.array_equal(fused.cpu().numpy(), alone.cpu().numpy(), equal_nan=True)
+    return {n: t.cpu().double().view(B, S, H, d).transpose(1, 2).numpy()
+            for n, t in (("o", o), ("dq", dq), ("dk", dk), ("dv", dv))}
+
+
+def _attention_rows64(q, k, v, do):
+    """One unit's causal attention in float64, each row over its visible keys
+    alone: (results, their sizes -- the same sums over magnitudes)."""
+    S, d = q.shape
+    z = lambda: np.zeros((S, d))  # noqa: E731
+    want, size = {n: z() for n in ("o", "dq", "dk", "dv")}, {n: z() for n in ("o", "dq", "dk", "dv")}
+    for i in range(S):
+        n = i + 1
+        s = k[:n] @ q[i] / 8.0
+        p = np.exp(s - s.max())
+        p /= p.sum()
+        dp = v[:n] @ do[i]
+        delta = float((p * dp).sum())
+        ds = p * (dp - delta) / 8.0
+        mag = p * (np.abs(v[:n]) @ np.abs(do[i]) + p @ (np.abs(v[:n]) @ np.abs(do[i]))) / 8.0
+        for name, w, m, x in (("o", p, p, v[:n]), ("dq", ds, mag, k[:n])):
+            want[name][i], size[name][i] = w @ x, m @ np.abs(x)
+        want["dk"][:n] += ds[:, None] * q[i]
+        size["dk"][:n] += mag[:, None] * np.abs(q[i])
+        want["dv"][:n] += p[:, None] * do[i]
+        size["dv"][:n] += p[:, None] * np.abs(do[i])
+    return want, size
+
+
+# What is planted, (tensor, row, dim, value): the largest floats, whose nearest
+# bf16 is an infinity; infinities and NaN; a key of the lowest value in one dim,
+# as a mask leaves it.  In the first and a later block, by the diagonal and far
+# from it.
+FMAX = float(np.finfo(np.float32).max)
+
+
+@pytest.mark.parametrize("plant", [
+    "v_max", "k_low", "q_max", "do_max", "v_inf", "k_inf", "q_inf", "do_inf", "v_nan", "do_nan"])
+@pytest.mark.parametrize("S,row", [(40, 17), (150, 70), (150, 3), (131, 130)])
+def test_exact_attention_takes_every_float(hip, torch_cuda, plant, S, row):
+    """The f32 family at head width 64 on operands whose bf16 parts overflow or
+    that are not finite: what float64 attention has finite is finite and within
+    1e-5 of the sum's size, element by element (an f32 rounding is 6e-8 of it);
+    what it has infinite is that infinity, what it has NaN is NaN.  Rows and
+    keys that do not see the planted one are as without it."""
+    B, H, d, dim = 1, 2, 64, 37
+    print(f"exact attention {plant} S={S} row={row}", flush=True)
+    r = rng(S + row)
+    x = {n: r.standard_normal((S, H * d)).astype(np.float32) for n in ("q", "k", "v", "do")}
+    name, kind = plant.split("_")
+    value = {"max": FMAX, "low": -FMAX, "inf": np.inf, "nan": np.nan}[kind]
+    at = dim + (d if H > 1 else 0)  # the second head
+    col = lambda n: x[n][:, at]  # noqa: E731
+    # The other side of the planted value's products: small where they would
+    # overflow f32 themselves, of one sign where a score goes to -inf.
+    if plant == "v_max":
+        col("do")[:] *= 1e-3
+    elif plant == "do_max":
+        col("v")[:] *= 1e-3
+    elif plant == "k_low":
+        col("q")[:] = np.abs(col("q")) + 0.5
+    elif plant == "k_inf":
+        value = -np.inf
+        col("q")[:] = np.abs(col("q")) + 0.5
+    elif plant == "q_max":  # the scores of one query stay within f32
+        col("k")[:] *= np.float32(1e-38)
+    x[name][row, at] = value
+    got = _exact_attention(hip, torch_cuda, *(x[n] for n in ("q", "k", "v", "do")), B, S, H)
+    bad = []
+    with np.errstate(all="ignore"):
+        for h in range(H):
+            want, size = _attention_rows64(*(x[n][:, h * d:(h + 1) * d].astype(np.float64)
+                                             for n in ("q", "k", "v", "do")))
+            for n in want:
+                g, w = got[n][0, h], want[n]
+                fin = np.isfinite(w) & (np.abs(w) < 0.99 * FMAX)
+                over = np.abs(size[n]) >= 0.99 * FMAX  # sums that pass through the f32 limit
+                ok = np.where(fin, np.abs(g - w) <= 1e-5 * size[n] + 1e-30,
+                              np.where(np.isnan(w), np.isnan(g), g == w))
+                ok |= over & np.isfinite(size[n])
+                if not ok.all():
+                    i, c = np.argwhere(~ok)[0]
+                    bad.append(f"{n} head {h}: {np.count_nonzero(~ok)} wrong, first at row {i} dim "
+                               f"{c}: {g[i, c]} for {w[i, c]} (size {size[n][i, c]:.3g})")
+    assert not bad, "; ".join(bad)
+
+
 # --- optimizer -----------------------------------------------------------------------------
 
 @pytest.mark.parametrize("n", [1, 2048, 100003])
