@@ -81,13 +81,16 @@ __device__ __forceinline__ Parts Split(const float (&x)[8]) {
   return r;
 }
 
-// hi += hh, lo += the five smaller part products.
+// hi += hh, lo += the five smaller part products, in an order that kSwap turns
+// with the operands' sides.
+template <bool kSwap = false>
 __device__ __forceinline__ void Mfma3(const Parts& a, const Parts& b, v16f& hi, v16f& lo) {
-  lo = Mfma(a.p[0], b.p[2], lo);
-  lo = Mfma(a.p[2], b.p[0], lo);
+  constexpr int kA = kSwap ? 2 : 0;
+  lo = Mfma(a.p[kA], b.p[2 - kA], lo);
+  lo = Mfma(a.p[2 - kA], b.p[kA], lo);
   lo = Mfma(a.p[1], b.p[1], lo);
-  lo = Mfma(a.p[0], b.p[1], lo);
-  lo = Mfma(a.p[1], b.p[0], lo);
+  lo = Mfma(a.p[kA / 2], b.p[1 - kA / 2], lo);
+  lo = Mfma(a.p[1 - kA / 2], b.p[kA / 2], lo);
   hi = Mfma(a.p[0], b.p[0], hi);
 }
 
@@ -141,12 +144,15 @@ __device__ __forceinline__ Parts ColParts(const Tile3& t, const FragOffsets& fo,
                 ColFrag(t.part[2], fo, dt, k0)}};
 }
 // Staged rows row0 .. + 32 against the own rows, over the 64 dims: lane (g, c)
-// gets rows 8q + 4g + e against own row c.
+// gets rows 8q + 4g + e against own row c.  kOwnKeys: the own rows are keys or
+// values (dK / dV), else the staged ones are; either way a query's and a key's
+// dot has the same bits, so dP - delta is 0 for a query that sees one key.
+template <bool kOwnKeys = false>
 __device__ __forceinline__ v16f Dot3(const Tile3& t, const FragOffsets& fo, int row0,
                                      const Parts (&own)[4]) {
   v16f hi = {}, lo = {};
 #pragma unroll
-  for (int s = 0; s < 4; ++s) Mfma3(RowParts(t, fo, row0, s), own[s], hi, lo);
+  for (int s = 0; s < 4; ++s) Mfma3<kOwnKeys>(RowParts(t, fo, row0, s), own[s], hi, lo);
   return hi + lo;
 }
 // acc[dt] += (the tile's columns 32 dt ..)^T over rows row0 .. + 32 times w,
@@ -560,7 +566,7 @@ Attn3DKDV(const float* __restrict__ q, const float* __restrict__ k, const float*
     for (int t = 0; t < 2; ++t) {
       const int it = i0 + 32 * t;
       if (it >= S || it + 31 < jw) continue;  // wave-uniform: no query sees a key
-      const v16f sc = Dot3(qt, fo, 32 * t, kf);
+      const v16f sc = Dot3<true>(qt, fo, 32 * t, kf);
       float p[16];
 #pragma unroll
       for (int r = 0; r < 16; ++r)
@@ -574,7 +580,7 @@ Attn3DKDV(const float* __restrict__ q, const float* __restrict__ k, const float*
       }
       if constexpr (kDV) Accum3(dt, fo, 32 * t, p, acc_v);
       if constexpr (kDK) {
-        const v16f dp = Dot3(dt, fo, 32 * t, vf);
+        const v16f dp = Dot3<true>(dt, fo, 32 * t, vf);
         float w[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r)

@@ -798,6 +798,21 @@ def test_exact_attention_takes_every_float(hip, torch_cuda, plant, S, row):
     assert not bad, "; ".join(bad)
 
 
+def test_exact_attention_passes_form_the_same_dots(hip, torch_cuda):
+    """Queries that see one key each: the forward has p = 1, dQ leaves delta =
+    dP, and dK / dV forms both dots again with the same bits -- dS = p (dP -
+    delta) is exactly 0, so dK is, and dV is exactly dO."""
+    B, S, H = 2, 203, 3
+    print("one visible key: dK, dV", flush=True)
+    r = rng(S)
+    q, k, v, do = (r.standard_normal((B * S, H * 64)).astype(np.float32) for _ in range(4))
+    at = np.tile(np.arange(S, dtype=np.int32), B)
+    got = _exact_attention(hip, torch_cuda, q, k, v, do, B, S, H, at)
+    assert not got["dk"].any(), "dK"
+    assert np.array_equal(got["dv"].transpose(0, 2, 1, 3).reshape(B * S, H * 64),
+                          do.astype(np.float64)), "dV"
+
+
 # --- optimizer -----------------------------------------------------------------------------
 
 @pytest.mark.parametrize("n", [1, 2048, 100003])
