@@ -179,6 +179,15 @@ __device__ __forceinline__ void Accum3(const Tile3& t, const FragOffsets& fo, in
 // maximum, so y log2(e) errs by 2^-24 of itself, as far as y's own rounding.
 __device__ __forceinline__ float ExpOf(float y) { return Exp2(y * kLog2e); }
 
+// In pairs: the sums of weights have few roundings, so that p's add up to 1 as
+// closely as they can (what is left over scales a component that all keys share).
+__device__ __forceinline__ float Sum16(const float (&x)[16]) {
+  float s[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) s[i] = x[2 * i] + x[2 * i + 1];
+  return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+}
+
 __device__ __forceinline__ void StoreRow(float* row, int g, const v16f (&acc)[2], float scale) {
 #pragma unroll
   for (int dt = 0; dt < 2; ++dt)
@@ -205,36 +214,29 @@ __device__ __forceinline__ void KeyBlocks(int start, int i0, int S, int& first, 
 // sees and no other: for the waves whose sums came out NaN.  Two lanes a row
 // (lane % 32), 32 of the 64 dims each; slow and rare.
 // ---------------------------------------------------------------------------
-struct Half {  // a lane's 32 dims of a row
-  float x[32];
-  __device__ __forceinline__ explicit Half(const float* row, int g) {
+struct Half {  // a lane's 32 dims of a row, StoreRow's
+  v16f x[2] = {};
+  Half() = default;
+  __device__ __forceinline__ Half(const float* row, int g) {
 #pragma unroll
     for (int e = 0; e < 32; e += 4) {
-      const float4 v = *reinterpret_cast<const float4*>(row + 32 * g + e);
-      x[e] = v.x, x[e + 1] = v.y, x[e + 2] = v.z, x[e + 3] = v.w;
+      const float4 v = *reinterpret_cast<const float4*>(row + 2 * e + 4 * g);
+      x[e / 16][e % 16] = v.x, x[e / 16][e % 16 + 1] = v.y;
+      x[e / 16][e % 16 + 2] = v.z, x[e / 16][e % 16 + 3] = v.w;
     }
-  }
-  __device__ __forceinline__ Half() {
-#pragma unroll
-    for (int e = 0; e < 32; ++e) x[e] = 0.0f;
   }
   // this += w r
   __device__ __forceinline__ void Add(float w, const Half& r) {
 #pragma unroll
-    for (int e = 0; e < 32; ++e) x[e] = __builtin_fmaf(w, r.x[e], x[e]);
-  }
-  __device__ __forceinline__ void Store(float* row, int g, float scale) const {
-#pragma unroll
-    for (int e = 0; e < 32; e += 4)
-      *reinterpret_cast<float4*>(row + 32 * g + e) =
-          make_float4(x[e] * scale, x[e + 1] * scale, x[e + 2] * scale, x[e + 3] * scale);
+    for (int e = 0; e < 32; ++e)
+      x[e / 16][e % 16] = __builtin_fmaf(w, r.x[e / 16][e % 16], x[e / 16][e % 16]);
   }
 };
 // The rows' dot over both lanes, the same in both.
 __device__ __forceinline__ float Dot(const Half& a, const Half& b) {
   float s = 0.0f;
 #pragma unroll
-  for (int e = 0; e < 32; ++e) s = __builtin_fmaf(a.x[e], b.x[e], s);
+  for (int e = 0; e < 32; ++e) s = __builtin_fmaf(a.x[e / 16][e % 16], b.x[e / 16][e % 16], s);
   return SwapSum(s);
 }
 
@@ -259,8 +261,8 @@ __device__ __forceinline__ void PlainFwd(const float* q_row, const float* k, con
     const float p = s == -INFINITY ? 0.0f : expf(s - mn);
     l = l * alpha + p;
     m = mn;
-#pragma unroll
-    for (int e = 0; e < 32; ++e) acc.x[e] *= alpha;
+    acc.x[0] *= alpha;
+    acc.x[1] *= alpha;
     acc.Add(p, Half(v + static_cast<size_t>(j) * ld, g));
   }
 }
@@ -379,15 +381,11 @@ Attn3Fwd(const float* __restrict__ q, const float* __restrict__ k, const float* 
     const float mn = fmaxf(m, SwapMax(mx));
     const float ref = mn == -INFINITY ? 0.0f : mn;
     const float alpha = m == -INFINITY ? 0.0f : ExpOf(m - ref);
-    float sum = 0.0f;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        p[t][r] = ExpOf(p[t][r] - ref);
-        sum += p[t][r];
-      }
-    l = l * alpha + sum;
+      for (int r = 0; r < 16; ++r) p[t][r] = ExpOf(p[t][r] - ref);
+    l = l * alpha + (Sum16(p[0]) + Sum16(p[1]));
     m = mn;
     acc[0] *= alpha;
     acc[1] *= alpha;
@@ -397,28 +395,36 @@ Attn3Fwd(const float* __restrict__ q, const float* __restrict__ k, const float* 
   }
   l = SwapSum(l);
   const size_t at = base + static_cast<size_t>(ic) * ld;
+  const auto store = [&](const v16f (&row)[2], float row_m, float row_l) {
+    if (i >= S) return;
+    const float inv = 1.0f / row_l;
+    StoreRow(o + at, g, row, inv);
+    if (g == 0)
+      *reinterpret_cast<float4*>(stats + (static_cast<size_t>(bh) * S + i) * 4) =
+          make_float4(row_m, inv, 0.0f, static_cast<float>(start));
+  };
   const bool plain = AnyNaN(acc, l != l);
-  Half row;
-  if (plain)
-    PlainFwd(q + at, k + base, v + base, ld, ic, start, WaveMinI(start), wave_last, g, row, m, l);
-  if (i >= S) return;
-  const float inv = 1.0f / l;
-  if (plain)
-    row.Store(o + at, g, inv);
-  else
-    StoreRow(o + at, g, acc, inv);
-  if (g == 0)
-    *reinterpret_cast<float4*>(stats + (static_cast<size_t>(bh) * S + i) * 4) =
-        make_float4(m, inv, 0.0f, static_cast<float>(start));
+  store(acc, m, l);
+  if (plain) {  // over the same addresses, lane by lane
+    Half row;
+    float row_m, row_l;
+    PlainFwd(q + at, k + base, v + base, ld, ic, start, WaveMinI(start), wave_last, g, row, row_m,
+             row_l);
+    store(row.x, row_m, row_l);
+  }
 }
 
 // ---------------------------------------------------------------------------
 // dQ (attention.cc:495-535) in one walk over the keys: dS = p (dP - delta) is
-// linear in delta, so dQ = (sum p dP k - delta sum p k) / sqrt(d) with delta =
-// sum p dP (in double) from the same walk -- four products and one exponential
-// a score where a walk for delta and one for dQ take five and two (395 us at
-// B8 H12 S1024, two walks, 224 us here), and its error against float64 stays
-// below half the f32 MFMA kernel's two-walk form's.
+// linear in delta, so dQ = (sum p (dP - ref) k - (delta - ref) sum p k) / sqrt(d)
+// for any ref, with delta = sum p dP (in double) from the same walk -- four
+// products and one exponential a score where a walk for delta and one for dQ
+// take five and two (395 us at B8 H12 S1024, two walks, 224 us here).  ref is
+// the mean of the dP met so far, weighted as delta weights them, and the sums
+// move with it, so what they hold is as small as dP - delta even where all keys
+// or values share a component (ref = 0 loses up to six times two walks' error
+// there, the first block's mean four).  A query that sees one key has ref =
+// delta = dP and dQ exactly 0.
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(kThreads, 1)
 Attn3DQ(const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
@@ -445,8 +451,9 @@ Attn3DQ(const float* __restrict__ q, const float* __restrict__ k, const float* _
   OwnParts(dout + base + static_cast<size_t>(ic) * ld, lane, df);
 
   const FragOffsets fo = MakeFragOffsets(lane);
-  v16f acc_d[2] = {}, acc_p[2] = {};  // sums of (p dP) k and of p k
-  double dsum = 0.0;
+  v16f acc_d[2] = {}, acc_p[2] = {};  // sums of p (dP - ref) k and of p k
+  double dsum = 0.0;                  // this half's sum of p dP
+  float psum = 0.0f, ref = 0.0f;
   Block3 nk, nv;
   nk.Load(k + base, ld, jb0 * kBlkRows, S);
   nv.Load(v + base, ld, jb0 * kBlkRows, S);
@@ -476,30 +483,41 @@ Attn3DQ(const float* __restrict__ q, const float* __restrict__ k, const float* _
         }
       }
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        w[r] = p[r] != 0.0f ? p[r] * dp[r] : 0.0f;
-        if (p[r] != 0.0f) dsum += static_cast<double>(dp[r]) * p[r];
-      }
+      for (int r = 0; r < 16; ++r) dsum += static_cast<double>(dp[r]) * p[r];
+      psum += Sum16(p);
+      // The weighted mean of the keys' dP so far; what is summed moves to it.
+      const float weight = SwapSum(psum), sum = SwapSum(static_cast<float>(dsum));
+      const float mean = weight > 0.0f ? sum / weight : ref;
+      const float move = mean - ref;
+      ref = mean;
+#pragma unroll
+      for (int dt = 0; dt < 2; ++dt) acc_d[dt] -= move * acc_p[dt];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) w[r] = p[r] * (dp[r] - ref);
       Accum3(kt, fo, 32 * t, w, acc_d);
       Accum3(kt, fo, 32 * t, p, acc_p);
     }
   }
-  float delta = static_cast<float>(dsum + __shfl_xor(dsum, 32, kWave));
+  dsum += __shfl_xor(dsum, 32, kWave);
+  float delta = static_cast<float>(dsum);
+  const float rest = static_cast<float>(dsum - static_cast<double>(ref));
   v16f acc[2];
 #pragma unroll
-  for (int dt = 0; dt < 2; ++dt) acc[dt] = (acc_d[dt] - delta * acc_p[dt]) * kIsd;
+  for (int dt = 0; dt < 2; ++dt) acc[dt] = (acc_d[dt] - rest * acc_p[dt]) * kIsd;
   const size_t at = base + static_cast<size_t>(ic) * ld;
+  const auto store = [&](const v16f (&row)[2], float row_delta) {
+    if (i >= S) return;
+    StoreRow(dq + at, g, row, 1.0f);
+    if (g == 0) stats[(static_cast<size_t>(bh) * S + i) * 4 + 2] = row_delta;
+  };
   const bool plain = AnyNaN(acc, delta != delta);
-  Half row;
-  if (plain)
+  store(acc, delta);
+  if (plain) {
+    Half row;
     PlainDQ(q + at, dout + at, k + base, v + base, ld, st.x, st.y, ic, start, WaveMinI(start),
             wave_last, g, row, delta);
-  if (i >= S) return;
-  if (plain)
-    row.Store(dq + at, g, 1.0f);
-  else
-    StoreRow(dq + at, g, acc, 1.0f);
-  if (g == 0) stats[(static_cast<size_t>(bh) * S + i) * 4 + 2] = delta;
+    store(row.x, delta);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -584,26 +602,24 @@ Attn3DKDV(const float* __restrict__ q, const float* __restrict__ k, const float*
         float w[16];
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          w[r] = p[r] != 0.0f ? (p[r] * (dp[r] - rows(sd, t, r))) * kIsd : 0.0f;
+          w[r] = (p[r] * (dp[r] - rows(sd, t, r))) * kIsd;
         Accum3(qt, fo, 32 * t, w, acc_k);
       }
     }
   }
   const size_t at = base + static_cast<size_t>(jc) * ld;
   const bool plain_k = kDK && AnyNaN(acc_k), plain_v = kDV && AnyNaN(acc_v);
-  Half row_k, row_v;
-  if (plain_k || plain_v)
+  if (j < S) {
+    if constexpr (kDK) StoreRow(dk + at, g, acc_k, 1.0f);
+    if constexpr (kDV) StoreRow(dv + at, g, acc_v, 1.0f);
+  }
+  if (plain_k || plain_v) {
+    Half row_k, row_v;
     PlainDKDV<kDK, kDV>(k + at, v + (kDK ? at : 0), q + base, dout + base, ld, st, jc, jw, S, g,
                         row_k, row_v);
-  if (j >= S) return;
-  if (plain_k)
-    row_k.Store(dk + at, g, 1.0f);
-  else if constexpr (kDK)
-    StoreRow(dk + at, g, acc_k, 1.0f);
-  if (plain_v)
-    row_v.Store(dv + at, g, 1.0f);
-  else if constexpr (kDV)
-    StoreRow(dv + at, g, acc_v, 1.0f);
+    if (plain_k && j < S) StoreRow(dk + at, g, row_k.x, 1.0f);
+    if (plain_v && j < S) StoreRow(dv + at, g, row_v.x, 1.0f);
+  }
 }
 
 dim3 GridOf(size_t B, size_t S, size_t H) {
