@@ -7,7 +7,7 @@
 //
 // Products.  Every f32 operand is split three ways, x = h + m + l, each part
 // the bf16 nearest to what is left: 8 + 8 + 8 significant bits, so the parts
-// hold x (to the last bit or so).  A product sums six of the nine part
+// hold x (to the last bit or so; below 2^-109 to 2^-134, where bf16 ends).  A product sums six of the nine part
 // products -- hh in the accumulator, hm, mh, mm, hl, lh in one of their own
 // that joins it at the end; the three left out are below 2^-26 of the operands'
 // product -- each exact in the MFMA, summed in f32.  Against float64 the
@@ -45,6 +45,9 @@
 
 namespace seeai {
 namespace {
+
+constexpr float kLog2eLo =  // log2(e) - kLog2e
+    static_cast<float>(1.4426950408889634074 - static_cast<double>(kLog2e));
 
 constexpr int kWaves = 4, kThreads = kWaves * kWave, kRowsWG = kWaves * 32;
 constexpr float kIsd = 0.125f;  // 1 / sqrt(64)
@@ -175,9 +178,17 @@ __device__ __forceinline__ void Accum3(const Tile3& t, const FragOffsets& fo, in
   }
 }
 
-// exp(y) by the hardware's exp2: y is a rounded difference from the row's
-// maximum, so y log2(e) errs by 2^-24 of itself, as far as y's own rounding.
-__device__ __forceinline__ float ExpOf(float y) { return Exp2(y * kLog2e); }
+// exp(y) for y <= 0 as 2^n 2^f, n the integer nearest to y log2(e) and f the
+// rest of it in two fused steps, so that it errs like expf (y = -75 .. 0: 3.5e-8
+// of itself in the mean square); 2^t of t = y log2(e) rounded errs by |y| 2^-24.
+// n is held at -200: -inf and all that is far below f32 give 0; NaN stays.  us,
+// forward / dQ / dK and dV at B8 H12 S1024: 107 / 231 / 243 here, 114 / 242 / 258
+// with expf and its range checks, 98 / 221 / 232 with 2^t.
+__device__ __forceinline__ float ExpOf(float y) {
+  const float n = fmaxf(__builtin_rintf(y * kLog2e), -200.0f);
+  const float f = __builtin_fmaf(y, kLog2eLo, __builtin_fmaf(y, kLog2e, -n));
+  return __builtin_amdgcn_ldexpf(Exp2(f), static_cast<int>(n));
+}
 
 // In pairs: the sums of weights have few roundings, so that p's add up to 1 as
 // closely as they can (what is left over scales a component that all keys share).

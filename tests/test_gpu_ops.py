@@ -868,6 +868,27 @@ def test_exact_attention_dq_with_common_offsets(hip, torch_cuda, k_mean, v_mean,
     assert err <= 4 * bar
 
 
+def test_exact_attention_weights_to_the_last_bits(hip, torch_cuda):
+    """A weight far below the row's largest is exp of its score to a few ulps:
+    scores that are exact (one dim, exactly held), two keys, the first with the
+    largest score and no value.  o = e / (1 + e) and dV's second row is that
+    times dO: an ulp of exp (2^-23) and at most six roundings."""
+    B, S, H = 1, 2, 256
+    r = rng(11)
+    # 19 bits; e^-75 is 2^-108.2, the least whose three bf16 parts hold 24 bits.
+    y = np.round(r.uniform(0.5, 75.0, H) * 2.0 ** 12) / 2.0 ** 12
+    q, k, v, do = (np.zeros((S, H, 64), np.float32) for _ in range(4))
+    q[:, :, 0] = 8.0
+    k[1, :, 0] = -y
+    v[1], do[1] = 1.0, 1.0
+    got = _exact_attention(hip, torch_cuda, *(t.reshape(S, H * 64) for t in (q, k, v, do)), B, S, H)
+    want = np.exp(-y) / (1.0 + np.exp(-y))
+    for name in ("o", "dv"):
+        e = np.abs(got[name][0, :, 1, :] / want[:, None] - 1.0).max()
+        print(f"  {name}: {e:.3g}", flush=True)
+        assert e <= 2.0 ** -23 + 6 * 2.0 ** -24, f"{name}: {e:.3g}"
+
+
 # --- optimizer -----------------------------------------------------------------------------
 
 @pytest.mark.parametrize("n", [1, 2048, 100003])
