@@ -303,8 +303,9 @@ XEntProbsKernel(const float* __restrict__ logits, const int32_t* __restrict__ la
 // Lane t holds float4 e T + t, e < kV, so (e, wave) is a segment of 256
 // consecutive columns and segments in order are the row.  The chain:
 //   1. every segment's plain sum, and their running sum P (one wave).  After n
-//      terms the serial sum is within n 2^-24 of the exact one; twice that
-//      around P bounds the binades a segment runs through.
+//      terms the serial sum is within n 2^-24 of the exact one, and P, a tree,
+//      within 20 2^-24; (n + 256) 2^-24 around P, n to the segment's end, bounds
+//      the binades a segment runs through.
 //   2. One binade and no tie: its terms rounded to that grid are summed.  Else
 //      the terms go to an LDS slot, and with one or two binades the running
 //      sums over the lanes on both grids and the lanes that hold a tie.
@@ -395,8 +396,10 @@ XEntRowKernel(const float* __restrict__ logits, const int32_t* __restrict__ labe
   if (wave == 0) {
     const int s0 = 2 * lane;
     const float a0 = s0 < kSegs ? ssum[s0] : 0.0f, a1 = s0 + 1 < kSegs ? ssum[s0 + 1] : 0.0f;
-    const float incl = WaveScan(a0 + a1);
-    const float p0 = incl - (a0 + a1), p1 = p0 + a0;  // the sum before each segment
+    // The sum before each segment: the lanes' before, not this lane's less its
+    // own, which would err by the size of what comes next.
+    const float before = __shfl_up(WaveScan(a0 + a1), 1, kWave);
+    const float p0 = lane > 0 ? before : 0.0f, p1 = p0 + a0;
     const auto info = [&](int s, float p, float a) {
       const float margin = static_cast<float>(s + 2) * 0x1p-16f;
       const float lo = p * (1.0f - margin), hi = (p + a) * (1.0f + margin);

@@ -530,6 +530,39 @@ def test_xent_rows_in_registers_keep_the_chain(hip, torch_cuda, C, kind):
     ctx.close()
 
 
+def test_xent_chain_before_a_jump_of_the_sum(hip, torch_cuda):
+    """Rows whose sum lies on a power of two (2^-10, within its own rounding)
+    after 512 terms, then takes 256 terms of a few steps of its grid, then the
+    row's largest two: which grid the 256 round to depends on the side of the
+    power the sum is on, and the probabilities are still bit for bit the serial
+    sum's."""
+    torch = torch_cuda
+    print("xent chain before a jump", flush=True)
+    N, C, k = 20000, 1024, -10
+    r = rng(5)
+    x = np.full((N, C), -60.0)
+    lead = r.standard_normal((N, 512)) * 0.05
+    x[:, :512] = lead + np.log(2.0 ** k / np.exp(lead).sum(axis=1, keepdims=True))
+    x[:, 512:768] = np.log(2.0 ** (k - 24) * r.uniform(0.3, 8, (N, 1)))
+    at = 768 + np.arange(N) % 255
+    x[np.arange(N), at] = 0.0
+    x[np.arange(N), at + 1] = np.log1p(-2.0 ** k * r.uniform(0.1, 0.9, N))
+    x = torch.from_numpy(x.astype(np.float32)).cuda()
+    labels = torch.zeros(N, dtype=torch.int32, device="cuda")
+    loss, probs = torch.full((1,), -1.0, device="cuda"), torch.full_like(x, -1.0)
+    ctx = hip.Context(0)
+    ctx.use_torch_stream()
+    ctx.call("seeai_xent_fwd", x.data_ptr(), labels.data_ptr(), loss.data_ptr(), probs.data_ptr(),
+             N, C, 0)
+    torch.cuda.synchronize()
+    ctx.close()
+    e = torch.exp(x - x.amax(dim=1, keepdim=True)).cpu().numpy()  # the same device expf
+    total = np.add.accumulate(e, axis=1, dtype=np.float32)[:, -1]
+    want = e * (np.float32(1.0) / total)[:, None]
+    wrong = np.flatnonzero((probs.cpu().numpy() != want).any(axis=1))
+    assert not wrong.size, f"{wrong.size} rows, the first {wrong[:4]}"
+
+
 @pytest.mark.parametrize("head,C", [("f32", 4000), ("q8", 4000), ("f32", 4004)])
 def test_head_product_leaves_the_loss_turns_row_maxima(hip, orc, backend, head, C):
     """A relaxed head product right before the loss turn leaves its logits'
