@@ -436,12 +436,13 @@ def test_xent(hip, orc, backend, N, C, masked):
 
 @pytest.mark.parametrize("masked", [False, True])
 @pytest.mark.parametrize("read_later", [False, True])
-@pytest.mark.parametrize("N,C", [(96, 1000), (32, 256), (1024, 16), (5, 3276)])
+@pytest.mark.parametrize("N,C", [(96, 1000), (32, 256), (1024, 16), (5, 3276), (38, 32772)])
 def test_xent_forward_fill_backward_fuse_bitwise(hip, orc, backend, masked, read_later, N, C):
     """The train program's loss turn -- softmax-xent forward, the fill of its
     seed, softmax-xent backward -- runs in a range as the fill and one pass
     that forms the probabilities and their gradient (a few rows: the whole
-    turn in one workgroup): bitwise the three run one by one, one fused
+    turn in one workgroup; past 32768 columns three passes over the logits):
+    bitwise the three run one by one, one fused
     dispatch; the probabilities stay unstored unless something after the
     backward reads them."""
     from tests.plan_ops import ins
@@ -563,15 +564,17 @@ def test_xent_chain_before_a_jump_of_the_sum(hip, torch_cuda):
     assert not wrong.size, f"{wrong.size} rows, the first {wrong[:4]}"
 
 
-@pytest.mark.parametrize("head,C", [("f32", 4000), ("q8", 4000), ("f32", 4004)])
-def test_head_product_leaves_the_loss_turns_row_maxima(hip, orc, backend, head, C):
-    """A relaxed head product right before the loss turn leaves its logits'
-    row maxima over 64-column groups in its epilogue; the turn forms each
-    row's max from them instead of a pass over the logits (fmax is exact and
-    order-free).  Bitwise the instructions one by one (the probabilities
-    unstored), at a vocabulary that is and one that is not a multiple of 64."""
+@pytest.mark.parametrize("head,N,C", [("f32", 300, 32832), ("q8", 300, 32832), ("f32", 130, 32836),
+                                      ("q8", 130, 32836)])
+def test_head_product_leaves_the_loss_turns_row_maxima(hip, orc, backend, head, N, C):
+    """A relaxed head product right before the loss turn, of rows longer than
+    the turn holds (32768 columns), leaves its logits' row maxima over 64-column
+    groups in its epilogue; the turn forms each row's max from them instead of a
+    pass over the logits (fmax is exact and order-free).  Bitwise the
+    instructions one by one (the probabilities unstored), at a vocabulary that
+    is and one that is not a multiple of 64, on 256 x 256 and 128 x 128 tiles."""
     from tests.plan_ops import ins
-    N, K = 2048, 256
+    K = 128
     r = rng(C + len(head))
     ar = Arena()
     x = ar.add("x", r.standard_normal((N, K)).astype(np.float32))
