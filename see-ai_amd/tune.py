@@ -45,7 +45,8 @@ ARMS = {
     "quantize_waves_per_cu": [4, 8, 16, 32],
     "relaxed_min_tiles_256": [1, 128, 256, 1 << 30],
     "relaxed_min_fill_256": [0, 50, 80, 95],
-    "relaxed_nt_dma_min_k": [256, 512, 768, 1024, 4096],
+    # Below 768 the field moves range fusions only, which no single product shows.
+    "relaxed_nt_dma_min_k": [768, 1024, 4096],
     "convert_wgs_per_cu": [2, 4, 8, 16, 32],
     "exact_longk_first": [1, 2],
     "relaxed_tile_192": [1, 2, 3],
@@ -171,8 +172,10 @@ class Bench:
                 yield f"relaxed q8 {'NT' if nt else 'NN'} {M}x{N}x{K}", setup
         elif field == "relaxed_nt_dma_min_k":
             # C4's dX products over f32 weights (K = 768 and 3072) and C5's
-            # q8 ones (K = 2048, 5632): NT, K either side of the threshold.
-            shapes = [("f32", 8192, 768, 768), ("f32", 8192, 3072, 768), ("f32", 8192, 768, 3072),
+            # q8 ones (K = 2048, 5632), and short K (every arm over 768 leaves
+            # those to the register-staged kernel): NT.
+            shapes = [("f32", 8192, 768, 768), ("f32", 2048, 1024, 256), ("f32", 8192, 3072, 768),
+                      ("f32", 8192, 768, 3072), ("f32", 8192, 2048, 512), ("q8", 2048, 1024, 256),
                       ("q8", 8192, 2048, 2048), ("q8", 8192, 5632, 2048)]
             if self.quick:
                 shapes = shapes[:2]
