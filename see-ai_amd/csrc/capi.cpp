@@ -391,20 +391,55 @@ bool ConvertedAlready(seeai_ctx* c, const GemmArgs& a, const seeai_ctx::CvtKey& 
   return true;
 }
 
+auto ShadowKey(const GemmArgs& a) {
+  return std::make_tuple(a.B, a.layout, a.b_kind, static_cast<uint64_t>(a.N),
+                         static_cast<uint64_t>(a.K));
+}
+
+// The weight's bf16 shadow, made on first use.
+hipError_t WeightShadow(seeai_ctx* c, const GemmArgs& a, void** shadow) {
+  if (auto it = c->shadows.find(ShadowKey(a)); it != c->shadows.end()) {
+    *shadow = it->second;
+    return hipSuccess;
+  }
+  if (hipError_t e = hipMalloc(shadow, a.N * Bf16DmaKp(a.K) * 2); e != hipSuccess) return e;
+  c->shadows[ShadowKey(a)] = *shadow;
+  return LaunchWeightShadow(a, *shadow, c->stream);
+}
+
+// Whether a product that the register-staged kernel, which needs no memory,
+// runs too (NT below the range fusions' K) has its shadow and its conversion
+// buffer, taken here where the device has the memory.  Not under a caller's
+// capture: nothing may be allocated there, and the caller's graph would name a
+// buffer that a later, larger product replaces (a range's own graphs are
+// dropped then).
+bool DmaMemory(seeai_ctx* c, const GemmArgs& a) {
+  const size_t need = a.M * Bf16DmaKp(a.K) * 2;
+  if (c->capturing) return c->shadows.count(ShadowKey(a)) && need <= c->cvt_bytes;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  void *shadow, *cvt;
+  bool ok = hipStreamIsCapturing(c->stream, &status) == hipSuccess &&
+            status == hipStreamCaptureStatusNone && WeightShadow(c, a, &shadow) == hipSuccess;
+  if (ok && need > c->cvt_bytes) {
+    ok = hipMalloc(&cvt, need) == hipSuccess;
+    if (ok) {  // grow after draining the stream
+      DropGraphs(c);
+      if (c->cvt) ok = hipStreamSynchronize(c->stream) == hipSuccess && hipFree(c->cvt) == hipSuccess;
+      c->cvt_key.at = nullptr;
+      c->cvt = cvt;
+      c->cvt_bytes = need;
+    }
+  }
+  if (!ok) (void)hipGetLastError();
+  return ok;
+}
+
 // The relaxed frozen-weight product on the bf16 direct-to-LDS kernel: the
-// weight's bf16 shadow (made once), A rounded into the workspace with its
+// weight's bf16 shadow, A rounded into the workspace with its
 // scales, then the GEMM and its epilogue.
 int GemmBf16Dma(seeai_ctx* c, GemmArgs& a, const char* what) {
-  const auto key = std::make_tuple(a.B, a.layout, a.b_kind, static_cast<uint64_t>(a.N),
-                                   static_cast<uint64_t>(a.K));
   void* shadow = nullptr;
-  if (auto it = c->shadows.find(key); it != c->shadows.end()) {
-    shadow = it->second;
-  } else {
-    SEEAI_TRY(c, hipMalloc(&shadow, a.N * Bf16DmaKp(a.K) * 2), "weight shadow alloc");
-    c->shadows[key] = shadow;
-    SEEAI_TRY(c, LaunchWeightShadow(a, shadow, c->stream), "weight shadow");
-  }
+  SEEAI_TRY(c, WeightShadow(c, a, &shadow), "weight shadow");
   const size_t need = a.M * Bf16DmaKp(a.K) * 2;
   // A copy a conversion sink left in one of the other slots.
   for (int s = 0; s < seeai_ctx::kXSlots; ++s)
@@ -436,7 +471,8 @@ int GemmBf16Dma(seeai_ctx* c, GemmArgs& a, const char* what) {
 // A GEMM launch with the workspace its kernel may use.
 int Gemm(seeai_ctx* c, GemmArgs& a, const char* what) {
   a.policy = &c->policy;
-  if (a.relaxed && c->allow_dma && Bf16DmaFitsAlone(a) && Immutable(c, a.B))
+  if (a.relaxed && c->allow_dma && Bf16DmaFitsAlone(a) && Immutable(c, a.B) &&
+      (Bf16DmaFits(a) || DmaMemory(c, a)))
     return GemmBf16Dma(c, a, what);
   if (const size_t bytes = a.relaxed ? 0 : GemmExactScratchBytes(a)) {
     void* ws;
@@ -2525,7 +2561,7 @@ namespace {
 // buffer and their weights' bf16 shadows are sized (and the shadows made)
 // here, so no instruction of the range drains the stream to allocate.
 int PresizeWorkspaces(seeai_ctx* c, const uint8_t* prog, uint64_t begin, uint64_t end) {
-  size_t scratch = 0, cvt = 0;
+  size_t scratch = 0, cvt = 0, cvt_alone = 0;  // cvt_alone: products that can do without
   for (uint64_t i = begin; i < end; ++i) {
     Instruction ins;
     std::memcpy(&ins, prog + i * sizeof(Instruction), sizeof ins);
@@ -2552,14 +2588,15 @@ int PresizeWorkspaces(seeai_ctx* c, const uint8_t* prog, uint64_t begin, uint64_
     a.relaxed = (ins.flags & kFlagRelaxed) && c->allow_relaxed ? 1 : 0;
     a.policy = &c->policy;
     if (a.relaxed && c->allow_dma && Bf16DmaFitsAlone(a) && Immutable(c, a.B)) {
-      cvt = std::max(cvt, static_cast<size_t>(a.M * Bf16DmaKp(a.K) * 2));
-      const auto key = std::make_tuple(a.B, a.layout, a.b_kind, static_cast<uint64_t>(a.N),
-                                       static_cast<uint64_t>(a.K));
-      if (c->shadows.find(key) == c->shadows.end()) {
-        void* shadow = nullptr;
-        SEEAI_TRY(c, hipMalloc(&shadow, a.N * Bf16DmaKp(a.K) * 2), "weight shadow alloc");
-        c->shadows[key] = shadow;
-        SEEAI_TRY(c, LaunchWeightShadow(a, shadow, c->stream), "weight shadow");
+      void* shadow;
+      const hipError_t e = WeightShadow(c, a, &shadow);
+      size_t& most = Bf16DmaFits(a) ? cvt : cvt_alone;
+      if (e == hipSuccess) {
+        most = std::max(most, static_cast<size_t>(a.M * Bf16DmaKp(a.K) * 2));
+      } else if (&most == &cvt) {
+        SEEAI_TRY(c, e, "weight shadow");
+      } else {
+        (void)hipGetLastError();
       }
     } else if (!a.relaxed) {
       scratch = std::max(scratch, GemmExactScratchBytes(a));
@@ -2569,14 +2606,20 @@ int PresizeWorkspaces(seeai_ctx* c, const uint8_t* prog, uint64_t begin, uint64_
     void* ws;
     if (int rc = Scratch(c, std::max(scratch, kInitialScratch), &ws)) return rc;
   }
-  if (cvt > c->cvt_bytes) {
+  if (const size_t want = std::max(cvt, cvt_alone); want > c->cvt_bytes) {
     DropGraphs(c);
     SEEAI_TRY(c, hipStreamSynchronize(c->stream), "conversion buffer drain");
     if (c->cvt) SEEAI_TRY(c, hipFree(c->cvt), "conversion buffer free");
     c->cvt = nullptr;
     c->cvt_bytes = 0;
-    SEEAI_TRY(c, hipMalloc(&c->cvt, cvt), "conversion buffer alloc");
-    c->cvt_bytes = cvt;
+    if (hipMalloc(&c->cvt, want) == hipSuccess) {
+      c->cvt_bytes = want;
+    } else {
+      (void)hipGetLastError();
+      c->cvt = nullptr;
+      if (cvt) SEEAI_TRY(c, hipMalloc(&c->cvt, cvt), "conversion buffer alloc");
+      c->cvt_bytes = cvt;
+    }
   }
   if (cvt > c->xcvt_bytes) {
     DropGraphs(c);

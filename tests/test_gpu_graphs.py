@@ -105,3 +105,56 @@ def test_a_policy_change_recaptures(hip, torch_cuda):
     assert graphed.graph_launches >= before + 2
     graphed.close()
     eager.close()
+
+
+@pytest.mark.parametrize("warm", [False, True])
+@pytest.mark.parametrize("kind", ["f32", "q8"])
+def test_a_short_k_product_under_a_callers_capture(hip, torch_cuda, kind, warm):
+    """A relaxed NT product of K below 768 while the caller captures its stream,
+    executed before or not: the library may take no memory there, so it is
+    recorded on the kernel that needs none, and every replay has the bits of the
+    product executed outside a capture, over inputs uploaded between."""
+    from tests.arena import Arena, f32_bits
+    from tests.conftest import bits_equal
+    from tests.plan_ops import ins
+    torch = torch_cuda
+    print(f"graphs: short-K product in a caller's capture, {kind} warm={warm}", flush=True)
+    M, N, K = 256, 384, 320
+    r = np.random.default_rng(5)
+    inputs = [r.standard_normal((M, K)).astype(np.float32) for _ in range(3)]
+    ar = Arena()
+    a = ar.add("A", inputs[0])
+    if kind == "q8":
+        w = ar.add("W", r.integers(-127, 128, (N, K)).astype(np.int8), rodata=True)
+        s = ar.add("ks", r.uniform(1e-3, 5e-2, K).astype(np.float32), rodata=True)
+        o = ar.empty("C", (M, N))
+        word = ins(30, [a, w, o, s], [M, N, K], flags=(1 << 5) | (1 << 4))
+    else:
+        w = ar.add("W", (r.standard_normal((N, K)) * 0.02).astype(np.float32), rodata=True)
+        o = ar.empty("C", (M, N))
+        word = ins(2, [a, w, o], [M, N, K], flags=1 << 5, imm=f32_bits(0.37))
+    arena, ro = ar.images()
+    captured, apart = hip.HipBackend(0), hip.HipBackend(0)
+    for be in (captured, apart):
+        be.Bind(arena.tobytes(), arena.nbytes, ro.tobytes())
+        be.Flush()
+    if warm:
+        captured.Execute(word)
+        captured.Flush()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured.ctx.use_torch_stream()
+        captured.Execute(word)
+    captured.ctx.use_torch_stream()
+    for x in inputs + inputs[:1]:
+        for be in (captured, apart):
+            be.Upload(a, x.tobytes())
+        apart.Execute(word)
+        apart.Flush()
+        graph.replay()
+        torch.cuda.synchronize()
+        got, want = (ar.get(np.frombuffer(be.Download(0, arena.nbytes), np.uint8), "C")
+                     for be in (captured, apart))
+        assert np.isfinite(want).all() and bits_equal(got, want)
+    captured.ctx.close()
+    apart.ctx.close()
