@@ -711,29 +711,61 @@ GemmI8DmaKernel(const int8_t* __restrict__ QA, const float* __restrict__ sa,
   // The products are C^T tiles (W fragments as the A operand): lane (h, lr)
   // holds columns n = 32 j + 8 q + 4 h + e, e < 4, of row m = 32 i + lr --
   // four consecutive floats of one C row, stored as 16 bytes straight from
-  // registers.
+  // registers.  Rows off 16 bytes go through LDS (the stages are done with) and
+  // leave a row's consecutive floats a wave: four-byte stores of a lane's own
+  // quad touch 32 rows each and took 98 us at 3500 x 5630 x 64, 45 here; 1004
+  // x 2902 x 304 20.0 and 12.5.
   const bool vec_out = (N % 4) == 0 && ((reinterpret_cast<uintptr_t>(C) |
                                          reinterpret_cast<uintptr_t>(sw) |
                                          reinterpret_cast<uintptr_t>(acc_out)) & 15) == 0;
   auto store = [&](int m, int n, float s_a, int a0, int a1, int a2, int a3) {
     const size_t at = static_cast<size_t>(m) * N + n;
-    if (vec_out && n + 3 < N) {
-      const float4 s4 = *reinterpret_cast<const float4*>(sw + n);
-      *reinterpret_cast<float4*>(C + at) =
-          make_float4((static_cast<float>(a0) * s_a) * s4.x, (static_cast<float>(a1) * s_a) * s4.y,
-                      (static_cast<float>(a2) * s_a) * s4.z, (static_cast<float>(a3) * s_a) * s4.w);
-      if (acc_out) *reinterpret_cast<int4*>(acc_out + at) = make_int4(a0, a1, a2, a3);
-    } else {
-      const int a[4] = {a0, a1, a2, a3};
+    if (n >= N) return;  // N % 4 == 0: whole quads
+    const float4 s4 = *reinterpret_cast<const float4*>(sw + n);
+    *reinterpret_cast<float4*>(C + at) =
+        make_float4((static_cast<float>(a0) * s_a) * s4.x, (static_cast<float>(a1) * s_a) * s4.y,
+                    (static_cast<float>(a2) * s_a) * s4.z, (static_cast<float>(a3) * s_a) * s4.w);
+    if (acc_out) *reinterpret_cast<int4*>(acc_out + at) = make_int4(a0, a1, a2, a3);
+  };
+  // The same quad into a staged row (and, rarely asked for, its accumulators).
+  auto stage_quad = [&](float* row, int m, int n, float s_a, int a0, int a1, int a2, int a3) {
+    const int a[4] = {a0, a1, a2, a3};
+    float c[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (n + e >= N) continue;
-        C[at + e] = (static_cast<float>(a[e]) * s_a) * sw[n + e];
-        if (acc_out) acc_out[at + e] = a[e];
-      }
-    }
+    for (int e = 0; e < 4; ++e) c[e] = (static_cast<float>(a[e]) * s_a) * sw[min(n + e, N - 1)];
+    *reinterpret_cast<float4*>(row) = make_float4(c[0], c[1], c[2], c[3]);
+    if (acc_out && m < M)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (n + e < N) acc_out[static_cast<size_t>(m) * N + n + e] = a[e];
   };
   if constexpr (KG == 1) {
+    if (!vec_out) {  // a wave's 32 rows at a time, through its own slice
+      constexpr int kLd = WN + 4;
+      static_assert(kWaves * 32 * kLd * 4 <= kStages * kStage, "rows fit");
+      __syncthreads();
+      float* rows = reinterpret_cast<float*>(smem) + wave * 32 * kLd;
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int mb = m0 + wm + i * 32;
+        const float s_a = sa[min(mb + lr, M - 1)];
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            stage_quad(rows + lr * kLd + j * 32 + 8 * q + 4 * h, mb + lr,
+                       n0 + wn + j * 32 + 8 * q + 4 * h, s_a, acc[i][j][4 * q],
+                       acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll 4
+        for (int x = lane; x < 32 * WN; x += kWave) {
+          const int m = mb + x / WN, n = n0 + wn + x % WN;
+          if (m < M && n < N) C[static_cast<size_t>(m) * N + n] = rows[x / WN * kLd + x % WN];
+        }
+        __builtin_amdgcn_wave_barrier();
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const int m = m0 + wm + i * 32 + lr;
@@ -752,6 +784,9 @@ GemmI8DmaKernel(const int8_t* __restrict__ QA, const float* __restrict__ sa,
     constexpr int kQuads = TM * TN * 4;
     static_assert(KG * kWaves * kQuads * kWave * 16 <= KG * kStages * kStage, "partials fit");
     static_assert(kQuads % KG == 0, "whole quads per group");
+    constexpr int kParts = KG * kWaves * kQuads * kWave * 16, kLd = BN + 4;
+    static_assert(kParts + BM * kLd * 4 <= KG * kStages * kStage, "rows fit");
+    float* const rows = reinterpret_cast<float*>(smem_all + kParts);
     __syncthreads();
     v4i* part = reinterpret_cast<v4i*>(smem_all);
 #pragma unroll
@@ -769,8 +804,17 @@ GemmI8DmaKernel(const int8_t* __restrict__ QA, const float* __restrict__ sa,
       v4i sum = part[(wave * kQuads + x) * kWave + lane];
 #pragma unroll
       for (int w = 1; w < KG; ++w) sum += part[((w * kWaves + wave) * kQuads + x) * kWave + lane];
-      const int m = m0 + wm + i * 32 + lr;
-      if (m < M) store(m, n0 + wn + j * 32 + 8 * q + 4 * h, sa[m], sum[0], sum[1], sum[2], sum[3]);
+      const int mr = wm + i * 32 + lr, m = m0 + mr, nr = wn + j * 32 + 8 * q + 4 * h;
+      if (!vec_out)
+        stage_quad(rows + mr * kLd + nr, m, n0 + nr, sa[min(m, M - 1)], sum[0], sum[1], sum[2], sum[3]);
+      else if (m < M)
+        store(m, n0 + nr, sa[m], sum[0], sum[1], sum[2], sum[3]);
+    }
+    if (vec_out) return;
+    __syncthreads();
+    for (int x = tid; x < BM * BN; x += KG * kWaves * kWave) {
+      const int m = m0 + x / BN, n = n0 + x % BN;
+      if (m < M && n < N) C[static_cast<size_t>(m) * N + n] = rows[x / BN * kLd + x % BN];
     }
   }
 }
