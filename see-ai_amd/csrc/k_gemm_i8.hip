@@ -552,7 +552,8 @@ __device__ __forceinline__ void WaitVm() {
   __builtin_amdgcn_s_waitcnt((n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14));
 }
 
-template <int BM, int BN, int kStages, int WGM, int WGN, int KG, bool kTail = true>
+template <int BM, int BN, int kStages, int WGM, int WGN, int KG, bool kTail = true,
+          bool kHeld = false>
 __global__ void __launch_bounds__(KG * WGM * WGN * kWave)
 GemmI8DmaKernel(const int8_t* __restrict__ QA, const float* __restrict__ sa,
                 const int8_t* __restrict__ QW, const float* __restrict__ sw,
@@ -681,32 +682,47 @@ GemmI8DmaKernel(const int8_t* __restrict__ QA, const float* __restrict__ sa,
     }
   };
 
-  // Every iteration loads one stage: past the last stage the loads repeat
-  // it (in bounds, into a buffer no later stage uses), so the number of
-  // stages in flight at each barrier is always kStages - 3.
+  // A K that the buffers hold whole (kHeld): every stage at once and one wait,
+  // 1 x 2048 x 512 3.4 -> 3.0 us.  Else every iteration loads one stage: past the
+  // last stage the loads repeat it (in bounds, into a buffer no later stage
+  // uses), so the number of stages in flight at each barrier is always kStages - 3.
   const int last = nsteps - 1;
+  if constexpr (kHeld) {  // last < kStages
 #pragma unroll
-  for (int s = 0; s < kStages - 1; ++s) issue(min(s, last), s);
-  WaitVm<(kStages - 2) * kPerStage>();
-  __builtin_amdgcn_s_barrier();
-  read(0, frag0, 0);
-  for (int it = 0; it < last; ++it) {
-    const int buf = it % kStages;
-    read(buf, frag1, 1);
+    for (int s = 0; s < kStages; ++s)
+      if (s <= last) issue(s, s);
+    WaitVm<0>();
+    __builtin_amdgcn_s_barrier();
+    for (int s = 0; s <= last; ++s) {
+      read(s, frag0, 0);
+      read(s, frag1, 1);
+      mfmas(0);
+      mfmas(1);
+    }
+  } else {
+#pragma unroll
+    for (int s = 0; s < kStages - 1; ++s) issue(min(s, last), s);
+    WaitVm<(kStages - 2) * kPerStage>();
+    __builtin_amdgcn_s_barrier();
+    read(0, frag0, 0);
+    for (int it = 0; it < last; ++it) {
+      const int buf = it % kStages;
+      read(buf, frag1, 1);
+      mfmas(0);
+      interleave(false);
+      WaitVm<(kStages - 3) * kPerStage>();
+      __builtin_amdgcn_s_barrier();
+      issue(min(it + kStages - 1, last), (it + kStages - 1) % kStages);
+      read((it + 1) % kStages, frag0, 0);
+      mfmas(1);
+      interleave(true);
+    }
+    read(last % kStages, frag1, 1);
     mfmas(0);
     interleave(false);
-    WaitVm<(kStages - 3) * kPerStage>();
-    __builtin_amdgcn_s_barrier();
-    issue(min(it + kStages - 1, last), (it + kStages - 1) % kStages);
-    read((it + 1) % kStages, frag0, 0);
     mfmas(1);
-    interleave(true);
+    WaitVm<0>();  // the repeated loads have landed before the workgroup ends
   }
-  read(last % kStages, frag1, 1);
-  mfmas(0);
-  interleave(false);
-  mfmas(1);
-  WaitVm<0>();  // the repeated loads have landed before the workgroup ends
 
   // The products are C^T tiles (W fragments as the A operand): lane (h, lr)
   // holds columns n = 32 j + 8 q + 4 h + e, e < 4, of row m = 32 i + lr --
@@ -837,11 +853,12 @@ int DeviceCUs() {
 
 namespace {
 
-enum class Tile { k32, k64Split, k64, k128, k256x128, k256 };
+enum class Tile { k32, k64Split, k64, k128, k256x128, k256, kStaged128 };
 
-// The direct-to-LDS tile for an M x N output: the one whose measured time at
-// its number of tiles per CU (x) is least.  A tile's time grows with K alike
-// for all of them, so K stays out.  Measured at K = 4096, us, MI355X:
+// The tile for an M x N output: the direct-to-LDS one whose measured time at
+// its number of tiles per CU (x) is least.  A tile's time grows with K much
+// alike for all of them, so K stays out but for the largest.  Measured at K =
+// 4096, us, MI355X:
 //
 //   tile (k-groups)    x <= 1               past that
 //   32 x 32 (4)        7.2                  11.2 at 2, 21.6 at 4
@@ -852,9 +869,12 @@ enum class Tile { k32, k64Split, k64, k128, k256x128, k256 };
 //   256 x 256          47 at 1/4, 50 at 1/2, 59.6 at 3/4, 73 at 1
 //
 // The two largest run one workgroup per CU, so they pay by whole rounds of
-// the CUs.  Register-staged tiles of 128 x 128 ran all of these
+// the CUs.  Over a short K a second round of 256 x 256 is mostly its C stores
+// with nothing beside them, and the register-staged 128 x 128 tiles are faster:
+// 3500 x 5632 (x = 1.2), K = 64 / 256 / 512 / 1024, 27.9 / 32.6 / 38.2 / 48.5 us
+// against 25.5 / 27.2 / 34.4 / 47.0.  Register-staged tiles of 128 x 128 ran all of these
 // before: 30-36 us for M from 65 to 1024 at 4096 x 4096, now 11-28.
-Tile PickTile(size_t M, size_t N) {
+Tile PickTile(size_t M, size_t N, size_t K) {
   const double cus = DeviceCUs();
   const auto x = [&](size_t bm, size_t bn) {
     return static_cast<double>((M + bm - 1) / bm) * static_cast<double>((N + bn - 1) / bn) / cus;
@@ -870,7 +890,11 @@ Tile PickTile(size_t M, size_t N) {
                       std::max(17.0 + 11.0 * x128, 23.5 * x128),
                       rounds(x(256, 128), 43.0, 20.0, 25.0),
                       rounds(x(256, 256), 73.0, 25.0, 48.0)};
-  return static_cast<Tile>(std::min_element(t, t + 6) - t);
+  const Tile best = static_cast<Tile>(std::min_element(t, t + 6) - t);
+  const double x256 = x(256, 256);
+  if (best == Tile::k256 && K <= 1024 && x256 > 1.0 && x256 != std::floor(x256))
+    return Tile::kStaged128;
+  return best;
 }
 
 }  // namespace
@@ -972,14 +996,22 @@ hipError_t LaunchGemmW8A8(const int8_t* QA, const float* sa, const int8_t* QWt, 
     hipLaunchKernelGGL((GemmI8TileKernel<128, 128, 128, 2, 2, true>), tiles(128, 128), dim3(256), 0,
                        s, QA, sa, QWt, sw, C, acc, m, n, static_cast<int64_t>(k), N);
   else
-    switch (big ? Tile::k256 : PickTile(M, N)) {
+    switch (big ? Tile::k256 : PickTile(M, N, K)) {
       case Tile::k32:
-        hipLaunchKernelGGL((GemmI8DmaKernel<32, 32, 6, 1, 1, 4>), tiles(32, 32), dim3(256), 0, s, QA,
-                           sa, QWt, sw, C, acc, m, n, k);
+        if (K <= 4 * 6 * kDmaBK)
+          hipLaunchKernelGGL((GemmI8DmaKernel<32, 32, 6, 1, 1, 4, true, true>), tiles(32, 32),
+                             dim3(256), 0, s, QA, sa, QWt, sw, C, acc, m, n, k);
+        else
+          hipLaunchKernelGGL((GemmI8DmaKernel<32, 32, 6, 1, 1, 4>), tiles(32, 32), dim3(256), 0, s,
+                             QA, sa, QWt, sw, C, acc, m, n, k);
         break;
       case Tile::k64Split:
-        hipLaunchKernelGGL((GemmI8DmaKernel<64, 64, 4, 2, 2, 2>), tiles(64, 64), dim3(512), 0, s, QA,
-                           sa, QWt, sw, C, acc, m, n, k);
+        if (K <= 2 * 4 * kDmaBK)
+          hipLaunchKernelGGL((GemmI8DmaKernel<64, 64, 4, 2, 2, 2, true, true>), tiles(64, 64),
+                             dim3(512), 0, s, QA, sa, QWt, sw, C, acc, m, n, k);
+        else
+          hipLaunchKernelGGL((GemmI8DmaKernel<64, 64, 4, 2, 2, 2>), tiles(64, 64), dim3(512), 0, s,
+                             QA, sa, QWt, sw, C, acc, m, n, k);
         break;
       case Tile::k64:
         hipLaunchKernelGGL((GemmI8DmaKernel<64, 64, 4, 2, 2, 1>), tiles(64, 64), dim3(256), 0, s, QA,
@@ -1000,6 +1032,10 @@ hipError_t LaunchGemmW8A8(const int8_t* QA, const float* sa, const int8_t* QWt, 
         else
           hipLaunchKernelGGL((GemmI8DmaKernel<256, 256, 4, 2, 4, 1>), tiles(256, 256), dim3(512), 0,
                              s, QA, sa, QWt, sw, C, acc, m, n, k);
+        break;
+      case Tile::kStaged128:
+        hipLaunchKernelGGL((GemmI8TileKernel<128, 128, 128, 2, 2, true>), tiles(128, 128), dim3(256),
+                           0, s, QA, sa, QWt, sw, C, acc, m, n, static_cast<int64_t>(k), N);
         break;
     }
   return hipGetLastError();

@@ -2318,13 +2318,16 @@ def test_w8a8_at_the_bench_shapes(hip, orc, torch_cuda, M):
 # Per direct-to-LDS tile (32, 64 with two k-groups, 64, 128, 256 x 128, 256): rows
 # and columns off the tile, K off the 64-byte stage; then any K and alignment
 # (64 and 128 tiles), down to one element.  Then each tile at a row length off 16
-# bytes (C's rows leave through LDS).
+# bytes (C's rows leave through LDS), the register-staged tiles of a short K past
+# one round of the largest, and the split tiles at the longest K they hold whole
+# and the next.
 @pytest.mark.parametrize("M,N,K,shift", [
     (1, 33, 16, 0), (63, 4095, 80, 0), (130, 4000, 1008, 0), (511, 4098, 144, 0),
     (500, 5632, 272, 0), (2047, 4094, 48, 0), (3000, 4001, 336, 0), (3000, 4001, 320, 0),
     (1, 1, 1, 0), (65, 63, 127, 0), (70, 66, 129, 0), (40, 130, 64, 3), (1500, 3002, 131, 0),
     (250, 4001, 1008, 0), (600, 3001, 96, 0), (1004, 2902, 304, 0), (2500, 3001, 48, 0),
-    (3500, 2901, 64, 0), (3500, 2901, 80, 0), (33, 102, 1600, 0), (130, 4001, 528, 0)])
+    (3500, 2901, 64, 0), (3500, 2901, 80, 0), (3500, 5632, 80, 0), (3500, 5630, 48, 0),
+    (33, 100, 1536, 0), (33, 102, 1600, 0), (130, 4000, 512, 0), (130, 4001, 528, 0)])
 def test_w8a8_tiles_and_ragged_rows(hip, torch_cuda, M, N, K, shift):
     """The int32 accumulators against an exact float64 product and C against
     its own expression, bit for bit; `shift` starts both operands that many
