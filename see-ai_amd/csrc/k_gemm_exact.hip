@@ -1704,14 +1704,17 @@ hipError_t LaunchFold(const GemmArgs& a, hipStream_t s) {
 
 // The chain kernel where the tiled kernel's grid would be small for the
 // reduction it carries: under 512 tiles of 64 x 64 and K above the panel.
-// NT's tiled kernel (32 x 64 blocks, eight chains an output) takes over
-// earlier: 512 x 2560 x 704, 320 blocks of 64 x 64, 136 us here and 115 there;
-// 512 x 768 x 768, 96 blocks, 33 and 59.  (Not where a block's columns or rows
-// are mostly past the output.)
+// NT's tiled kernel (32 x 64 blocks, eight chains an output) fills its rounds of
+// the CUs worse but takes any K alike, where the chain kernel's last chunk of 128
+// goes term by term at about seven times the cost: f32, chain / tiled, us, 336
+// blocks of 64 x 64 at K = 768 91 / 122, 1024 114 / 160, 1001 195 / 161; 404 at
+// 4096 553 / 628, 1001 240 / 160; 456 at 640 107 / 104, 4096 662 / 634.  (Not
+// where a block's columns or rows are mostly past the output.)
 bool Chain(const GemmArgs& a) {
   const size_t tiles = ((a.M + 63) / 64) * ((a.N + 63) / 64);
-  const bool whole = a.M >= 64 && a.N >= 64;
-  return a.K > static_cast<size_t>(kPanelK) && tiles < (a.layout == 1 && whole ? 320 : 512);
+  if (a.K <= static_cast<size_t>(kPanelK) || tiles >= 512) return false;
+  if (a.layout != 1 || a.M < 64 || a.N < 64 || tiles < 320) return true;
+  return tiles * (a.K + 6 * (a.K % kChainK)) < 430 * a.K;
 }
 
 template <int kLayout, int kBKind, int BM, int BN>
