@@ -1708,13 +1708,20 @@ hipError_t LaunchFold(const GemmArgs& a, hipStream_t s) {
 // the CUs worse but takes any K alike, where the chain kernel's last chunk of 128
 // goes term by term at about seven times the cost: f32, chain / tiled, us, 336
 // blocks of 64 x 64 at K = 768 91 / 122, 1024 114 / 160, 1001 195 / 161; 404 at
-// 4096 553 / 628, 1001 240 / 160; 456 at 640 107 / 104, 4096 662 / 634.  (Not
-// where a block's columns or rows are mostly past the output.)
+// 4096 553 / 628, 1001 240 / 160; 456 at 640 107 / 104, 4096 662 / 634.  Narrow
+// weights cost the tiled kernel more: int8, 342 at 2048 185 / 294, 438 at
+// 2255 492 / 698; bf16, 440 at 1252 184 / 196.  (Not where a block's columns or rows are
+// mostly past the output.)
+// NN / TN of a K up to the panel's, where the panel kernel stops: below 224
+// blocks, panel / tiled / chain, us: TN 496 x 956 x 304 17.4 / 22.0 / 14.1, NN
+// 2669 x 130 x 363 24.2 / 26.4 / 13.7.
 bool Chain(const GemmArgs& a) {
   const size_t tiles = ((a.M + 63) / 64) * ((a.N + 63) / 64);
-  if (a.K <= static_cast<size_t>(kPanelK) || tiles >= 512) return false;
+  if (a.K <= static_cast<size_t>(kPanelK)) return a.layout != 1 && a.K >= 64 && tiles < 224;
+  if (tiles >= 512) return false;
   if (a.layout != 1 || a.M < 64 || a.N < 64 || tiles < 320) return true;
-  return tiles * (a.K + 6 * (a.K % kChainK)) < 430 * a.K;
+  const size_t most = a.b_kind == 0 ? 430 : a.b_kind == 1 ? 700 : 600;
+  return tiles * (a.K + 6 * (a.K % kChainK)) < most * a.K;
 }
 
 template <int kLayout, int kBKind, int BM, int BN>
@@ -1790,12 +1797,18 @@ size_t Tiles64(const GemmArgs& a) { return ((a.M + 63) / 64) * ((a.N + 63) / 64)
 // (below, the rows kernel and the small-output routes are faster: 1024 x 512
 // x 512, 128 blocks of 64 x 64, 44 us against 27), and not so many that the
 // 64 x 64 tiles' lower LDS traffic counts (2048 x 32000 x 768: 2339 us
-// against 2096; 8192 x 768 x 768, 1536 blocks: 225 / 222).
+// against 2096; 8192 x 768 x 768, 1536 blocks: 225 / 222).  f32 weights: nor just
+// past 2048 of them, two a SIMD, where they pay for four and the 64 x 64 tiles, a
+// block per CU and round, for three (2672 x 772 x 988, 2100 and 546: 102 / 87;
+// 804 x 3528 x 760, 2886 and 728: 79 / 71; but 4352 x 772 x 1236, 884: 131 / 142;
+// int8 904 x 2572 x 992, 615: 110 / 114).
 // Past the panel's K the chain kernel is what it replaces, whose time goes with
 // the outputs, so a narrow product needs as many of them (N = 32, K = 768,
 // here / chain: M = 12800 64 / 51, 25600 66 / 83; K = 2048 164 / 130, 167 /
 // 212).
 bool Tile(const GemmArgs& a) {
+  const size_t tiles32 = ((a.M + kTile - 1) / kTile) * ((a.N + kTile - 1) / kTile);
+  if (a.b_kind == 0 && tiles32 > 2048 && Tiles64(a) <= 768) return false;
   return TileFits(a) && a.M >= kTile && a.N >= kTile && Tiles64(a) >= 200 && Tiles64(a) < 1024 &&
          (a.K <= static_cast<size_t>(kPanelK) || a.M * a.N >= size_t{200} * 64 * 64);
 }
@@ -1814,9 +1827,15 @@ hipError_t LaunchTile(const GemmArgs& a, hipStream_t s) {
 // 28, 1024 x 256 x 256 15 / 10.5, 2048 x 128 x 128 9.3 / 7.0, 512 x 768 x 768
 // 39 (chain) / 33, 8 x 32000 x 768 40 / 31; but 256 x 768 x 768 (48 blocks) 21
 // / 26, 64 x 256 x 256 (4) 8.8 / 9.3.  Not over long K, where the chain kernel's
-// LDS serves it better: 5120 x 64 x 768 35 / 30, x 2048 88 / 108.
+// LDS serves it better: x 2048 at 5120 x 64 88 / 108; past the panel's K not with
+// a second column group mostly empty (4448 x 80 x 540 19.4 / 20.5) nor, bf16, a
+// few rows (18 x 5840 x 664 12.7 / 16.7).  Not int8 weights, a byte a lane and
+// load with its scale: 76 x 1612 x 364 17 / 61, 68 x 4248 x 700 40 / 116.
 bool Rows(const GemmArgs& a) {
-  if (a.layout != 0 || a.K < 4 || a.K > 1024 || a.K % 4 != 0 || a.alpha_a != 1.0f || a.a_k_scale || a.N < 64)
+  if (a.layout != 0 || a.b_kind == 1 || a.K < 4 || a.K > 1024 || a.K % 4 != 0 ||
+      a.alpha_a != 1.0f || a.a_k_scale || a.N < 64)
+    return false;
+  if (a.K > static_cast<size_t>(kPanelK) && ((a.N < 128 && a.N % 64 != 0) || (a.b_kind == 2 && a.M < 32)))
     return false;
   const size_t t = Tiles64(a);
   return t >= (a.K <= static_cast<size_t>(kPanelK) ? 32u : 80u) && (t < 200 || a.M < kTile);
@@ -1841,10 +1860,12 @@ hipError_t LaunchRows(const GemmArgs& a, hipStream_t s) {
 // x 16 blocks count: NN 8192 x 12 x 256, 512 of them, 11 / 31; 8192 x 24 x 512
 // (1024) 47 / 58; 16384 x 24 (2048) 14 / 18 at K = 128, 32 / 32 at 256, 93 / 59
 // at 512.  NT's rows of eight lanes gain less from it: 8192 x 24 (1024) 17 /
-// 22 at K = 256, 56 / 40 at 512; 8192 x 12 x 512 (512) 24 / 40.
+// 22 at K = 256, 56 / 40 at 512; 8192 x 12 x 512 (512) 24 / 40.  NN / TN below 224
+// blocks of 64 x 64 and K = 64 stay too (688 x 600 x 48 4.0 / 6.1).
 bool Panel(const GemmArgs& a) {
   if (a.K == 0 || a.K > static_cast<size_t>(kPanelK) || (a.M + 15) / 16 > 65535) return false;
-  if (a.M <= 16 || Tiles64(a) < 100) return true;
+  if (a.M <= 32 || Tiles64(a) < 100) return true;
+  if (a.layout != 1 && a.K < 64 && Tiles64(a) < 224) return true;
   const size_t blocks = ((a.M + 15) / 16) * ((a.N + 15) / 16);
   if (a.layout == 1) return blocks <= 1024 && blocks * a.K <= 327680;
   return blocks <= (a.K <= 256 ? 2048 : 1024);
