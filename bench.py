@@ -287,7 +287,7 @@ def main():
         "config": {"workload": "W8A8 GEMM M=4096 K=4096 N=4096 (BASELINE configs[1])",
                    "M": M, "N": N, "K": K, "parallelism": "single GPU"},
         "roofline": {
-            "kernel": "GemmI8DmaKernel<4,2,4>",
+            "kernel": "GemmI8DmaKernel<256,256,4,2,4,1,false>",
             "bound": "mfma",
             "achieved": round(achieved, 1),
             "peak": PEAK_INT8_TOPS,

@@ -7,8 +7,8 @@
 //
 // Products.  Every f32 operand is split three ways, x = h + m + l, each part
 // the bf16 nearest to what is left: 8 + 8 + 8 significant bits, so the parts
-// hold x (to the last bit or so; below 2^-109 to 2^-134, where bf16 ends).  A product sums six of the nine part
-// products -- hh in the accumulator, hm, mh, mm, hl, lh in one of their own
+// hold x (to the last bit or so; below 2^-109 to 2^-134, where bf16 ends).  A
+// product sums six of the nine part products -- hh in the accumulator, hm, mh, mm, hl, lh in one of their own
 // that joins it at the end; the three left out are below 2^-26 of the operands'
 // product -- each exact in the MFMA, summed in f32.  Against float64 the
 // results are as close as sums of v_mfma_f32_16x16x4f32 (a chain of rounded
@@ -16,23 +16,24 @@
 // bf16 products take 3/8 of the f32 MFMA's time, which bounded these kernels
 // (v_mfma_f32_16x16x4f32 at 55-60 % of its rate).  us, f32 MFMA / here:
 //
-//   B8 H12 S1024     forward 184 / 108   dQ 408 / 224    dK + dV 342 / 270
-//   B16 H16 S2048            1491 / 878     3627 / 1805          3258 / 2245
-//   B1 H8 S328                 43 / 26        94 / 40              65 / 51
+//   B8 H12 S1024     forward 175 / 114   dQ 414 / 240    dK + dV 350 / 258
+//   B16 H16 S2048            1517 / 894     3626 / 2129          3229 / 2232
+//   B1 H8 S328                 43 / 28        95 / 42              66 / 47
 //
-// 2-norm error against float64 at B2 H4 S1024, unit normals, f32 MFMA / here:
-// O 3.2e-7 / 1.4e-7, dQ 3.9e-7 / 1.8e-7, dK 7.6e-7 / 3.1e-7, dV 7.4e-7 /
-// 3.1e-7; with scores of standard deviation 8, dQ 1.9e-6 / 9.9e-7.  What bounds
-// them now is a wave's own chain (products, exps, splits) at two waves a SIMD
-// (one for dQ and dK / dV): MFMA busy 23 %, VALU 32 % of the forward.
+// 2-norm error against float64 at H4 S2048, f32 MFMA / here: unit normals O
+// 4.0e-7 / 1.7e-7, dQ 4.6e-7 / 2.1e-7, dK 1.1e-6 / 4.3e-7, dV 1.1e-6 / 4.4e-7;
+// scores of standard deviation 8, dQ 1.9e-6 / 7.9e-7; means of 3 in K and V, dQ
+// 8.7e-6 / 7.3e-6.  What bounds them now is a wave's own chain (products, exps,
+// splits) at 1.4 waves a SIMD (0.9 for dQ and dK / dV): MFMA busy 32 / 31 / 28 %,
+// VALU 49 / 41 / 34 % of the forward, dQ, dK / dV at B8 H12 S1024.
 //
 // Geometry.  A workgroup of four waves owns 128 rows of one (b, h) -- queries
 // for the forward and dQ, keys for dK / dV -- each wave 32 of them, their parts
 // held as MFMA fragments.  The other side streams in 64-row blocks, split once
 // as it is staged into three bf16 tiles in LDS; one buffer (48 KiB for the
 // pair) and the next block in flight in registers, so two of the forward's
-// workgroups share a CU and one multiplies while the other stages.  Tiles, fragments and the
-// transposed score layout are k_attn16.hip's.
+// workgroups share a CU and one multiplies while the other stages.  Tiles,
+// fragments and the transposed score layout are k_attn16.hip's.
 //
 // An infinity, a NaN, or a float past the largest bf16 (3.3895e38) has no such
 // parts: its last one is NaN, and with it every sum it joins.  A wave whose sums
@@ -433,9 +434,9 @@ Attn3Fwd(const float* __restrict__ q, const float* __restrict__ k, const float* 
 // take five and two (395 us at B8 H12 S1024, two walks, 224 us here).  ref is
 // the mean of the dP met so far, weighted as delta weights them, and the sums
 // move with it, so what they hold is as small as dP - delta even where all keys
-// or values share a component (ref = 0 loses up to six times two walks' error
-// there, the first block's mean four).  A query that sees one key has ref =
-// delta = dP and dQ exactly 0.
+// or values share a component (emulated, ref = 0 errs up to seven times as far as
+// two walks there, the first block's mean up to six, the running mean as far).
+// A query that sees one key has ref = delta = dP and dQ exactly 0.
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(kThreads, 1)
 Attn3DQ(const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,

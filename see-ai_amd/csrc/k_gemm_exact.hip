@@ -241,8 +241,9 @@ __global__ void __launch_bounds__(kThreads) GemmExactKernel(GemmArgs g) {
 // per one-wave workgroup, 4 x 4 outputs a lane, so 2048 x 768 outputs are six
 // waves a CU rather than one and a half 64 x 64 workgroups.  The chains are
 // VALU work -- four multiplies and four adds a quad and output, no
-// contraction -- which the kernel reaches 85 % of the measured rate of (two
-// VALU operations a product: about 50 TFLOP/s) where the waves divide evenly.  K moves 16 at
+// contraction -- and the kernel issues one VALU instruction a SIMD every four
+// cycles where its waves divide evenly (2048 x 768 x 3072; 1.5 for
+// GemmExactKernel's four waves a SIMD at 8192 x 2048 x 512).  K moves 16 at
 // a time through two LDS buffers (k-major), the next step's operands in
 // flight in registers as they were loaded: the scales apply at the LDS store,
 // so no load is waited for before the step's arithmetic.  Larger register
