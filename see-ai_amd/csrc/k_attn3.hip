@@ -8,12 +8,12 @@
 // Products.  Every f32 operand is split three ways, x = h + m + l, each part
 // the bf16 nearest to what is left: 8 + 8 + 8 significant bits, so the parts
 // hold x (to the last bit or so; below 2^-109 to 2^-134, where bf16 ends).  A
-// product sums six of the nine part products -- hh in the accumulator, hm, mh, mm, hl, lh in one of their own
-// that joins it at the end; the three left out are below 2^-26 of the operands'
-// product -- each exact in the MFMA, summed in f32.  Against float64 the
-// results are as close as sums of v_mfma_f32_16x16x4f32 (a chain of rounded
-// f32 terms) or closer: fewer roundings at the accumulator's magnitude.  Six
-// bf16 products take 3/8 of the f32 MFMA's time, which bounded these kernels
+// product sums six of the nine part products -- hh in the accumulator, hm, mh,
+// mm, hl, lh in one of their own that joins it at the end; the three left out are
+// below 2^-26 of the operands' product -- each exact in the MFMA, summed in f32.
+// Against float64 the results are as close as sums of v_mfma_f32_16x16x4f32 (a
+// chain of rounded f32 terms) or closer: fewer roundings at the accumulator's
+// magnitude.  Six bf16 products take 3/8 of the f32 MFMA's time, which bounded these kernels
 // (v_mfma_f32_16x16x4f32 at 55-60 % of its rate).  us, f32 MFMA / here:
 //
 //   B8 H12 S1024     forward 175 / 114   dQ 414 / 240    dK + dV 350 / 258
