@@ -206,7 +206,10 @@ typedef struct seeai_tile_policy {
                                      this percent full (<= 100) */
   uint32_t relaxed_nt_dma_min_k;  /* relaxed NT on rodata weights: the direct-to-LDS kernel's
                                      range fusions from this K (default 768); a value over 768
-                                     also keeps the register-staged kernel below it */
+                                     also keeps the register-staged kernel below it.  Up to
+                                     768 a product by itself runs the direct-to-LDS kernel from
+                                     K = 64 where its memory (the weight's bf16 copy, a buffer
+                                     for A) can be had and the caller captures no stream */
   uint32_t convert_wgs_per_cu;    /* workgroups per CU of the relaxed GEMMs' activation
                                      conversion (default 8, <= 64) */
   uint32_t exact_longk_first;     /* exact skinny long-K GEMM: 1 the two-pass form before the
