@@ -115,6 +115,10 @@ __device__ __forceinline__ float WaveScan(float v) {
   v = DppAdd<0x142, 0xa>(v);  // lane 15 of a row to the next row
   return DppAdd<0x143, 0xc>(v);  // lane 31 to the upper half
 }
+// The lane before's value, 0 in lane 0 (wave_shr 1).
+__device__ __forceinline__ float WaveShift(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, false));
+}
 __device__ __forceinline__ float ReadLane(float v, int lane) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
@@ -398,8 +402,7 @@ XEntRowKernel(const float* __restrict__ logits, const int32_t* __restrict__ labe
     const float a0 = s0 < kSegs ? ssum[s0] : 0.0f, a1 = s0 + 1 < kSegs ? ssum[s0 + 1] : 0.0f;
     // The sum before each segment: the lanes' before, not this lane's less its
     // own, which would err by the size of what comes next.
-    const float before = __shfl_up(WaveScan(a0 + a1), 1, kWave);
-    const float p0 = lane > 0 ? before : 0.0f, p1 = p0 + a0;
+    const float p0 = WaveShift(WaveScan(a0 + a1)), p1 = p0 + a0;
     const auto info = [&](int s, float p, float a) {
       const float margin = static_cast<float>(s + 2) * 0x1p-16f;
       const float lo = p * (1.0f - margin), hi = (p + a) * (1.0f + margin);
