@@ -1865,7 +1865,7 @@ hipError_t LaunchRows(const GemmArgs& a, hipStream_t s) {
 // blocks of 64 x 64 and K = 64 stay too (688 x 600 x 48 4.0 / 6.1).
 bool Panel(const GemmArgs& a) {
   if (a.K == 0 || a.K > static_cast<size_t>(kPanelK) || (a.M + 15) / 16 > 65535) return false;
-  if (a.M <= 32 || Tiles64(a) < 100) return true;
+  if (a.M <= 16 || Tiles64(a) < 100) return true;
   if (a.layout != 1 && a.K < 64 && Tiles64(a) < 224) return true;
   const size_t blocks = ((a.M + 15) / 16) * ((a.N + 15) / 16);
   if (a.layout == 1) return blocks <= 1024 && blocks * a.K <= 327680;
