@@ -1713,12 +1713,16 @@ hipError_t LaunchFold(const GemmArgs& a, hipStream_t s) {
 // weights cost the tiled kernel more: int8, 342 at 2048 185 / 294, 438 at
 // 2255 492 / 698; bf16, 440 at 1252 184 / 196.  (Not where a block's columns or rows are
 // mostly past the output.)
-// NN / TN of a K up to the panel's, where the panel kernel stops: below 224
-// blocks, panel / tiled / chain, us: TN 496 x 956 x 304 17.4 / 22.0 / 14.1, NN
-// 2669 x 130 x 363 24.2 / 26.4 / 13.7.
+// NN / TN of a K up to the panel's, where the panel kernel stops: up to 768
+// blocks of 32 x 32, three a CU, panel / tiled / chain, us: TN 496 x 956 x 304
+// 17.4 / 22.0 / 14.1, NN 2669 x 130 x 363 24.2 / 26.4 / 13.7, 6075 x 128 x 501
+// (760 blocks) 140 / 58 / 51; but 7035 x 128 x 257 (880) 56 / 33 / 39, and below
+// K = 160 the chunk is mostly fill: 6075 x 128 x 131 19.6 / 19.0 / 20.0, x 65
+// 11.1 / 11.5 / 12.4.
 bool Chain(const GemmArgs& a) {
   const size_t tiles = ((a.M + 63) / 64) * ((a.N + 63) / 64);
-  if (a.K <= static_cast<size_t>(kPanelK)) return a.layout != 1 && a.K >= 64 && tiles < 224;
+  if (a.K <= static_cast<size_t>(kPanelK))
+    return a.layout != 1 && a.K >= 160 && ((a.M + 31) / 32) * ((a.N + 31) / 32) <= 768;
   if (tiles >= 512) return false;
   if (a.layout != 1 || a.M < 64 || a.N < 64 || tiles < 320) return true;
   const size_t most = a.b_kind == 0 ? 430 : a.b_kind == 1 ? 700 : 600;
@@ -1829,16 +1833,18 @@ hipError_t LaunchTile(const GemmArgs& a, hipStream_t s) {
 // 39 (chain) / 33, 8 x 32000 x 768 40 / 31; but 256 x 768 x 768 (48 blocks) 21
 // / 26, 64 x 256 x 256 (4) 8.8 / 9.3.  Not over long K, where the chain kernel's
 // LDS serves it better: x 2048 at 5120 x 64 88 / 108; past the panel's K not with
-// a second column group mostly empty (4448 x 80 x 540 19.4 / 20.5) nor, bf16, a
-// few rows (18 x 5840 x 664 12.7 / 16.7).  Not int8 weights, a byte a lane and
+// a second column group mostly empty (chain / rows: 4448 x 80 x 764 38 / 44, 6000
+// x 80 x 1000 67 / 76; but 6000 x 112 x 520 52 / 36) nor, bf16, a few rows of few
+// blocks (18 x 5840 x 640, 92 blocks, 19 / 25; 18 x 8000, 125, 31 / 25; 18 x 32000
+// 88 / 44).  Not int8 weights, a byte a lane and
 // load with its scale: 76 x 1612 x 364 17 / 61, 68 x 4248 x 700 40 / 116.
 bool Rows(const GemmArgs& a) {
   if (a.layout != 0 || a.b_kind == 1 || a.K < 4 || a.K > 1024 || a.K % 4 != 0 ||
       a.alpha_a != 1.0f || a.a_k_scale || a.N < 64)
     return false;
-  if (a.K > static_cast<size_t>(kPanelK) && ((a.N < 128 && a.N % 64 != 0) || (a.b_kind == 2 && a.M < 32)))
-    return false;
   const size_t t = Tiles64(a);
+  if (a.K > static_cast<size_t>(kPanelK) && ((a.N < 96 && a.N != 64) || (a.b_kind == 2 && a.M < 32 && t < 112)))
+    return false;
   return t >= (a.K <= static_cast<size_t>(kPanelK) ? 32u : 80u) && (t < 200 || a.M < kTile);
 }
 
@@ -1862,13 +1868,17 @@ hipError_t LaunchRows(const GemmArgs& a, hipStream_t s) {
 // (1024) 47 / 58; 16384 x 24 (2048) 14 / 18 at K = 128, 32 / 32 at 256, 93 / 59
 // at 512.  NT's rows of eight lanes gain less from it: 8192 x 24 (1024) 17 /
 // 22 at K = 256, 56 / 40 at 512; 8192 x 12 x 512 (512) 24 / 40.  NN / TN below 224
-// blocks of 64 x 64 and K = 64 stay too (688 x 600 x 48 4.0 / 6.1).
+// blocks of 64 x 64 stay while their blocks times K are few: 688 x 600 x 48 4.0 /
+// 6.1, 7035 x 90 x 64 (2640 blocks) 9.1 / 10.8, x 130 16.1 / 18.5, 6075 x 128 x
+// 130 (3040) 17.4 / 18.5; but 7035 x 128 x 65 (3520) 12.4 / 11.7, x 131 22.7 / 19.0; f32 NN
+// with more columns than rows, half as many: 48 x 13001 x 131 (2439) 24.3 / 18.3.
 bool Panel(const GemmArgs& a) {
   if (a.K == 0 || a.K > static_cast<size_t>(kPanelK) || (a.M + 15) / 16 > 65535) return false;
   if (a.M <= 16 || Tiles64(a) < 100) return true;
-  if (a.layout != 1 && a.K < 64 && Tiles64(a) < 224) return true;
   const size_t blocks = ((a.M + 15) / 16) * ((a.N + 15) / 16);
   if (a.layout == 1) return blocks <= 1024 && blocks * a.K <= 327680;
+  const bool wide_f32 = a.b_kind == 0 && a.layout == 0 && a.N > a.M;
+  if (Tiles64(a) < 224 && blocks <= 3072 && blocks * a.K <= 3072 * (wide_f32 ? 65 : 130)) return true;
   return blocks <= (a.K <= 256 ? 2048 : 1024);
 }
 

@@ -279,13 +279,16 @@ def test_gemm_narrow_weights(hip, orc, backend, M, N, K):
 # The 32 x 32 one-wave tiles (200 to 1023 blocks of 64 x 64, whole float4
 # rows), the rows kernel (fewer, or few rows) and, past the panel kernel, the
 # general tiled kernel (rows off float4): off every tile, K off the 16-deep step.
-# Then the dispatch's other edges: the chain kernel at K up to the panel's (under
-# 224 blocks) and, NT, at 320 to 511 blocks over whole and ragged chunks; the
-# panel below K = 64; 64 x 64 tiles for just over 2048 of 32 x 32 (f32 weights).
+# Then the dispatch's other edges: the chain kernel at K up to the panel's (up
+# to 768 blocks of 32 x 32) and, NT, at 320 to 511 blocks over whole and ragged
+# chunks; the panel at short K past 100 blocks; 64 x 64 tiles for just over 2048
+# of 32 x 32 (f32 weights); the rows kernel past the panel's K with few bf16 rows
+# and with a second column group partly empty.
 TILES_AND_ROWS = [(830, 1100, 68), (803, 1028, 44), (515, 260, 36), (5, 4100, 20),
                   (640, 524, 524), (806, 1030, 67), (500, 956, 304), (2669, 130, 363),
                   (1284, 1060, 516), (1281, 1057, 520), (1281, 1057, 641), (690, 602, 48),
-                  (2180, 992, 520), (24, 6500, 70)]
+                  (2180, 992, 520), (24, 6500, 70), (1203, 601, 100), (1203, 601, 162),
+                  (18, 8200, 520), (5200, 100, 520)]
 
 
 @pytest.mark.parametrize("M,N,K", TILES_AND_ROWS)
